@@ -65,6 +65,44 @@ def test_quantize_bit_exact_vs_oracle(gpu, M, K, R, G, iters, sample, dt):
     assert np.array_equal(got, oIDX), f"indices: {np.mean(got != oIDX):.2e} differ"
 
 
+# (M, K, rows_per_cb, scale_group, iters, sample, weights): cell lists of both
+# grid sizes and the full scan, one and several partial sums a block, a partial
+# last block, and weights whose points crowd a few places (equal centroids,
+# full lists, cell borders, the square's corners)
+CELL_CASES = [
+    (512, 512, 512, 512, 4, 9000, "normal"),
+    (1000, 512, 256, 32, 2, 40_000, "normal"),
+    (1024, 512, 1024, 64, 3, 200_000, "normal"),
+    (512, 512, 512, 32, 3, 9000, "three"),
+    (512, 512, 512, 32, 3, 9000, "grid"),
+    (512, 512, 512, 512, 3, 20_000, "outlier"),
+    (512, 512, 512, 512, 0, 9000, "outlier"),
+    (256, 256, 256, 256, 3, 2048, "tight"),
+    (256, 256, 256, 256, 3, 2047, "tight"),
+]
+
+
+@pytest.mark.parametrize("M,K,R,G,iters,sample,kind", CELL_CASES)
+def test_quantize_cells_bit_exact_vs_oracle(gpu, M, K, R, G, iters, sample, kind):
+    W = weights(M, K, M + K + iters)
+    rng = np.random.default_rng(9)
+    if kind == "three":
+        W = rng.choice(np.float32([-0.01, 0.0, 0.02]), (M, K))
+    elif kind == "grid":  # multiples of 1/64 of the scale: on cell borders
+        W = (rng.integers(-64, 65, (M, K)) / 64).astype(np.float32)
+    elif kind == "outlier":  # one large weight a row: the points crowd the middle
+        W[:, 0] = 5.0
+    elif kind == "tight":  # all points within a few cells of the corners
+        W = np.sign(W) * (1 - 0.05 * rng.random((M, K))).astype(np.float32)
+    IDX, Cb, S = quantize_gpu(gpu, torch.from_numpy(W).to(gpu), M, K, R, G, iters, sample, 31)
+    oIDX, oCb, oS, _ = oracle.vq_quantize(W, oracle.F32, M, K, R, G, iters=iters, sample=sample,
+                                          seed=31)
+    assert np.array_equal(host_bits(S, np.uint16), oS), "scales"
+    assert np.array_equal(host_bits(Cb, np.uint16), oCb), "codebooks"
+    got = IDX.cpu().numpy()
+    assert np.array_equal(got, oIDX), f"indices: {np.mean(got != oIDX):.2e} differ"
+
+
 def test_quantize_zero_and_constant_rows(gpu):
     """All-zero groups (scale 0, pairs divided by 1) and constant rows."""
     M, K = 64, 128
