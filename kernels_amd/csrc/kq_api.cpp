@@ -338,9 +338,10 @@ kq_status kq_moe_down_combine(const uint8_t* pool, const kq_moe_desc* d, const u
     if (!aligned(pool, 16) || !aligned(H, 16) || !aligned(idx, 4) || !aligned(wgt, 4))
         return KQ_EALIGN;
     if (!aligned(Y, y_dtype == KQ_F32 ? 4 : 2)) return KQ_EALIGN;
-    (void)ws;  // the combine happens in LDS
-    (void)ws_bytes;
-    return hip_status(kq::launch_moe_down(pool, *d, idx, wgt, H, Y, y_dtype == KQ_F32, batch,
+    // per-slot products go to the workspace where there is one (a missing,
+    // small or misaligned one is no error: the combine then happens in LDS)
+    if (check_ws(d, batch, ws, ws_bytes) != KQ_OK) ws = nullptr;
+    return hip_status(kq::launch_moe_down(pool, *d, idx, wgt, H, Y, y_dtype == KQ_F32, batch, ws,
                                           reinterpret_cast<hipStream_t>(stream)));
 }
 

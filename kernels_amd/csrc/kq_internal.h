@@ -80,7 +80,7 @@ hipError_t launch_moe_gate_up(const uint8_t* pool, const kq_moe_desc& d, const u
                               const uint16_t* xh, uint16_t* H, uint32_t batch, hipStream_t s);
 hipError_t launch_moe_down(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                            const float* wgt, const uint16_t* H, void* Y, bool y_f32,
-                           uint32_t batch, hipStream_t s);
+                           uint32_t batch, void* ws, hipStream_t s);  // ws: workspace or null
 // Router logits only (float [batch][n_experts] to lg; xh = half(X) if X is fp32).
 hipError_t launch_moe_logits(const void* R, bool r_f32, const void* X, bool x_f32, uint32_t batch,
                              const kq_moe_desc& d, uint16_t* xh, float* lg, hipStream_t s);

@@ -1525,7 +1525,42 @@ __device__ __forceinline__ PartRange part_range(const Plan& ps, uint32_t nslots,
     return PartRange{s, e - s};
 }
 
-// Gate/up + SwiGLU, partitioned by expert (3-16 tokens): workgroup b
+// The plan of a caller's idx for the partitioned kernels. An entry takes at
+// most one slot per token there (LDS blocks, lanes of a store); a caller may
+// name an expert twice for one token, and an entry with more slots than tokens
+// is cut into entries of at most `batch` slots (all threads; at most nslots
+// entries in all).
+__device__ void plan_from_idx(const uint32_t* idx, uint32_t batch, uint32_t TK, uint32_t NE,
+                              Plan& ps, uint32_t* s_idx, uint32_t* bits) {
+    const uint32_t tid = threadIdx.x, nslots = batch * TK;
+    if (tid < nslots) s_idx[tid] = idx[tid];
+    __syncthreads();
+    build_plan(s_idx, nslots, NE, ps, bits);
+    const bool over = tid < ps.n && (uint32_t)(__popcll(ps.mask[tid][0]) +
+                                               __popcll(ps.mask[tid][1])) > batch;
+    if (!__syncthreads_or(over)) return;
+    if (tid == 0) {
+        uint32_t n = ps.n;
+        for (uint32_t u = 0; u < n; ++u) {  // an entry's rest becomes the entry behind the last
+            uint64_t a = ps.mask[u][0], b = ps.mask[u][1], m[2] = {0, 0};
+            for (uint32_t k = 0; k < batch && (a | b) != 0; ++k) {
+                const uint32_t sl = pop_slot(a, b);
+                m[sl >> 6] |= 1ull << (sl & 63);
+            }
+            ps.mask[u][0] = m[0];
+            ps.mask[u][1] = m[1];
+            if ((a | b) == 0) continue;
+            ps.expert[n] = ps.expert[u];
+            ps.mask[n][0] = a;
+            ps.mask[n][1] = b;
+            ++n;
+        }
+        ps.n = n;
+    }
+    __syncthreads();
+}
+
+// Gate/up + SwiGLU, partitioned by expert (2-16 tokens): workgroup b
 // streams the row chunk part_assign gives it of one plan entry's expert
 // (half 0 the gate row, half 1 the up row) with only the x vectors of that
 // expert's tokens in LDS, and writes h for each of its slots. Each expert's
@@ -1540,11 +1575,12 @@ __device__ __forceinline__ PartRange part_range(const Plan& ps, uint32_t nslots,
 // LDS; workgroup 0 publishes idx, wgt and the plan for the down launch.
 // Every token's x is loaded at entry, right after the wave's logits, and
 // staged in LDS by token, so the staging never waits behind the weight ring.
-template <int J>
+// IDX (the standalone entry point): the routing is the caller's, in idx_out.
+template <int J, bool IDX>
 __global__ __launch_bounds__(64 * kStWaves) void moe_gu_part_k(
     const uint8_t* __restrict__ pool, kq_moe_desc d, const uint16_t* __restrict__ xh,
-    uint32_t batch, uint16_t* __restrict__ H, const float* __restrict__ lg,
-    uint32_t* __restrict__ idx_out, float* __restrict__ wgt_out, Plan* __restrict__ plan_out) {
+    uint32_t batch, uint16_t* __restrict__ H, const float* __restrict__ lg, uint32_t* idx_out,
+    float* __restrict__ wgt_out, Plan* __restrict__ plan_out) {
     extern __shared__ __align__(16) unsigned char act[];  // [batch x blocks], by token
     __shared__ Plan ps;
     __shared__ uint32_t s_idx[kMaxSlots];
@@ -1561,25 +1597,30 @@ __global__ __launch_bounds__(64 * kStWaves) void moe_gu_part_k(
     // logits go first, so the top-k waits for them alone (loads retire in
     // order) and not for the x of every token; every wave loads both sets
     // (clamped to a valid token), so the wait counts are exact.
-    const uint32_t NE = d.n_experts;
-    float lgv[2][4];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const uint32_t t = min(wave + r * kStWaves, batch - 1);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) lgv[r][q] = lg[(size_t)t * NE + min(lane + 64 * q, NE - 1)];
-    }
     StStage st;
-    st_stage_load(st, xh, batch, K);
-    // 2. top-k of every token, then the plan
+    if constexpr (IDX) {
+        st_stage_load(st, xh, batch, K);
+        plan_from_idx(idx_out, batch, TK, d.n_experts, ps, s_idx, bits);
+    } else {
+        const uint32_t NE = d.n_experts;
+        float lgv[2][4];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const uint32_t t = wave + r * kStWaves;
-        if (t < batch) topk_vals(lgv[r], NE, TK, s_idx + t * TK, s_wgt + t * TK);  // uniform
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t t = min(wave + r * kStWaves, batch - 1);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) lgv[r][q] = lg[(size_t)t * NE + min(lane + 64 * q, NE - 1)];
+        }
+        st_stage_load(st, xh, batch, K);
+        // 2. top-k of every token, then the plan
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t t = wave + r * kStWaves;
+            if (t < batch) topk_vals(lgv[r], NE, TK, s_idx + t * TK, s_wgt + t * TK);  // uniform
+        }
+        __syncthreads();
+        build_plan(s_idx, batch * TK, d.n_experts, ps, bits);
+        if (blockIdx.x == 0) publish_plan(ps, s_idx, s_wgt, batch * TK, idx_out, wgt_out, plan_out);
     }
-    __syncthreads();
-    build_plan(s_idx, batch * TK, d.n_experts, ps, bits);
-    if (blockIdx.x == 0) publish_plan(ps, s_idx, s_wgt, batch * TK, idx_out, wgt_out, plan_out);
     // 3. this workgroup's range of (plan entry u, row i) items, u-major: from
     // 8 tokens equal-cost ranges (a range may span entries), below that the
     // whole-workgroup split of part_assign (one entry per workgroup, so every
@@ -1751,17 +1792,24 @@ __global__ __launch_bounds__(64 * kStWaves) void moe_gu_part_k(
 // (Combining in the last workgroup of each row chunk instead measured slower:
 // 125 us per block at 8 tokens with device-coherent stores, 130 with fences,
 // against 119 with the separate launch.)
-template <int J>
+// IDX (the standalone entry point): the plan is built from the caller's idx.
+template <int J, bool IDX>
 __global__ __launch_bounds__(64 * kStWaves) void moe_dn_part_k(
     const uint8_t* __restrict__ pool, kq_moe_desc d, const float* __restrict__ wgt,
-    const Plan* __restrict__ plan_g, const uint16_t* __restrict__ H, uint32_t nslots,
-    float* __restrict__ ys) {
+    const Plan* __restrict__ plan_g, const uint32_t* __restrict__ idx,
+    const uint16_t* __restrict__ H, uint32_t nslots, float* __restrict__ ys) {
     extern __shared__ __align__(16) unsigned char act[];  // [nvec h blocks]
     __shared__ uint32_t s_next;  // next row pair of the workgroup's range to hand out
     const uint32_t HID = d.hidden, K = d.inter, nw = K >> 3, nch = K >> 5;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t half = lane >> 5, rowb = K >> 1, metab = (K >> 6) * 2;
+    if constexpr (IDX) {
+        __shared__ Plan ps;
+        __shared__ uint32_t s_idx[kMaxSlots], bits[8];
+        plan_from_idx(idx, nslots / d.top_k, d.top_k, d.n_experts, ps, s_idx, bits);
+        plan_g = &ps;
+    }
     const PartAssign pa = part_assign(plan_g, nslots, HID >> 1, d.n_experts);
     if (pa.u == 0xFFFFFFFFu) return;  // uniform: no share of the plan
     const uint32_t ex = pa.ex;
@@ -2527,31 +2575,33 @@ hipError_t launch_gu_st(const uint8_t* pool, const kq_moe_desc& d, const uint32_
 
 // One round: one workgroup per CU (the partitioned kernels run one 8-wave
 // workgroup per CU at their register use), and at least one per plan entry.
-uint32_t part_grid(const kq_moe_desc& d, uint32_t batch) {
+// (idx: a caller's routing, whose entries may be cut, see plan_from_idx).
+uint32_t part_grid(const kq_moe_desc& d, uint32_t batch, bool idx) {
     const uint32_t nslots = batch * d.top_k;
-    const uint32_t nu = nslots < d.n_experts ? nslots : d.n_experts;  // plan entries at most
+    const uint32_t nu = idx || nslots < d.n_experts ? nslots : d.n_experts;  // plan entries at most
     return cu_count() > nu ? cu_count() : nu;
 }
 
-template <int J>
+template <int J, bool IDX>
 hipError_t go_gu_part(const uint8_t* pool, const kq_moe_desc& d, const uint16_t* xh, uint16_t* H,
                       uint32_t batch, GuTopk tk, hipStream_t s) {
-    auto kern = moe_gu_part_k<J>;
+    auto kern = moe_gu_part_k<J, IDX>;
     const size_t lds = st_act_bytes(batch, d.hidden);  // every token's x
     const hipError_t e = st_lds(kern, lds);
     if (e != hipSuccess) return e;
-    kern<<<part_grid(d, batch), 64 * kStWaves, lds, s>>>(pool, d, xh, batch, H, tk.lg, tk.idx,
-                                                          tk.wgt, tk.plan);
+    kern<<<part_grid(d, batch, IDX), 64 * kStWaves, lds, s>>>(pool, d, xh, batch, H, tk.lg, tk.idx,
+                                                               tk.wgt, tk.plan);
     return hipGetLastError();
 }
 
+template <bool IDX>
 hipError_t launch_gu_part(const uint8_t* pool, const kq_moe_desc& d, const uint16_t* xh,
                           uint16_t* H, uint32_t batch, GuTopk tk, hipStream_t s) {
     switch (chunks_j(d.hidden)) {
-        case 1: return go_gu_part<1>(pool, d, xh, H, batch, tk, s);
-        case 2: return go_gu_part<2>(pool, d, xh, H, batch, tk, s);
-        case 3: return go_gu_part<3>(pool, d, xh, H, batch, tk, s);
-        case 4: return go_gu_part<4>(pool, d, xh, H, batch, tk, s);
+        case 1: return go_gu_part<1, IDX>(pool, d, xh, H, batch, tk, s);
+        case 2: return go_gu_part<2, IDX>(pool, d, xh, H, batch, tk, s);
+        case 3: return go_gu_part<3, IDX>(pool, d, xh, H, batch, tk, s);
+        case 4: return go_gu_part<4, IDX>(pool, d, xh, H, batch, tk, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -2567,6 +2617,13 @@ template <bool FP>
 hipError_t launch_gu(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                      const Plan* plan, const uint16_t* xh, uint16_t* H, uint32_t batch,
                      hipStream_t s) {
+    if constexpr (!FP) {
+        // the block's choice (block_gu_streams); 16 tokens at gpt-oss-120b
+        // shapes: per tile 147 us, partitioned 87 us
+        if (!block_gu_streams(d, batch) && gu_part_ok(d, batch))
+            return launch_gu_part<true>(pool, d, xh, H, batch,
+                                        GuTopk{nullptr, const_cast<uint32_t*>(idx), nullptr, nullptr}, s);
+    }
     if (gu_streams(d, batch))
         return launch_gu_st<FP ? 1 : 0>(pool, d, idx, plan, xh, H, batch, GuTopk{}, s);
     switch (chunks_j(d.hidden)) {
@@ -2579,16 +2636,16 @@ hipError_t launch_gu(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* 
 }
 
 // One round of cost-weighted row chunks (part_assign), then the combine.
-template <int J>
-hipError_t go_dn_part(const uint8_t* pool, const kq_moe_desc& d, const float* wgt,
-                      const Plan* plan, const uint16_t* H, void* Y, bool y_f32, uint32_t batch,
+template <int J, bool FP>
+hipError_t go_dn_part(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
+                      const float* wgt, const Plan* plan, const uint16_t* H, void* Y, bool y_f32, uint32_t batch,
                       float* ys, hipStream_t s) {
-    auto kern = moe_dn_part_k<J>;
+    auto kern = moe_dn_part_k<J, !FP>;
     const uint32_t nslots = batch * d.top_k;
     const size_t lds = st_act_bytes(batch, d.inter);  // at most one slot per token per expert
     hipError_t e = st_lds(kern, lds);
     if (e != hipSuccess) return e;
-    kern<<<part_grid(d, batch), 64 * kStWaves, lds, s>>>(pool, d, wgt, plan, H, nslots, ys);
+    kern<<<part_grid(d, batch, !FP), 64 * kStWaves, lds, s>>>(pool, d, wgt, plan, idx, H, nslots, ys);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const uint32_t n = batch * d.hidden;
     moe_combine_k<<<(n + 255) / 256, 256, 0, s>>>(ys, Y, y_f32 ? 1 : 0, batch, d.top_k, d.hidden);
@@ -2599,7 +2656,7 @@ hipError_t go_dn_part(const uint8_t* pool, const kq_moe_desc& d, const float* wg
 // stages), inter <= one word per thread, the h blocks in LDS.
 bool dn_part_ok(const kq_moe_desc& d, uint32_t batch) {
     return batch <= (uint32_t)kStXr && (d.inter >> 3) <= 64u * kStWaves &&
-           d.blob < (1ull << 31) && st_act_bytes(batch, d.inter) + 1024 <= kLdsMax;
+           d.blob < (1ull << 31) && st_act_bytes(batch, d.inter) + kStStatic <= kLdsMax;
 }
 
 // ys: workspace for the per-slot products (nullptr: not available).
@@ -2609,15 +2666,13 @@ hipError_t launch_dn(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* 
                      uint32_t batch, hipStream_t s, float* ys = nullptr) {
     const uint32_t nslots = batch * d.top_k, npairs = d.hidden / 2;
     const uint32_t pp = (npairs + cu_count() - 1) / cu_count();
-    if constexpr (FP) {
-        if (ys && !st_ok(d, nslots, d.inter, (size_t)nslots * 2 * pp * 4) && dn_part_ok(d, batch)) {
-            switch (chunks_j(d.inter)) {
-                case 1: return go_dn_part<1>(pool, d, wgt, plan, H, Y, y_f32, batch, ys, s);
-                case 2: return go_dn_part<2>(pool, d, wgt, plan, H, Y, y_f32, batch, ys, s);
-                case 3: return go_dn_part<3>(pool, d, wgt, plan, H, Y, y_f32, batch, ys, s);
-                case 4: return go_dn_part<4>(pool, d, wgt, plan, H, Y, y_f32, batch, ys, s);
-                default: return hipErrorInvalidValue;
-            }
+    if (ys && !st_ok(d, nslots, d.inter, (size_t)nslots * 2 * pp * 4) && dn_part_ok(d, batch)) {
+        switch (chunks_j(d.inter)) {
+            case 1: return go_dn_part<1, FP>(pool, d, idx, wgt, plan, H, Y, y_f32, batch, ys, s);
+            case 2: return go_dn_part<2, FP>(pool, d, idx, wgt, plan, H, Y, y_f32, batch, ys, s);
+            case 3: return go_dn_part<3, FP>(pool, d, idx, wgt, plan, H, Y, y_f32, batch, ys, s);
+            case 4: return go_dn_part<4, FP>(pool, d, idx, wgt, plan, H, Y, y_f32, batch, ys, s);
+            default: return hipErrorInvalidValue;
         }
     }
     if (st_ok(d, nslots, d.inter, (size_t)nslots * 2 * pp * 4)) {
@@ -2805,8 +2860,10 @@ hipError_t launch_moe_gate_up(const uint8_t* pool, const kq_moe_desc& d, const u
 
 hipError_t launch_moe_down(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                            const float* wgt, const uint16_t* H, void* Y, bool y_f32,
-                           uint32_t batch, hipStream_t s) {
-    return launch_dn<false>(pool, d, idx, wgt, nullptr, H, Y, y_f32, batch, s);
+                           uint32_t batch, void* ws, hipStream_t s) {
+    float* ys = ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + ws_layout(d, batch).ys)
+                   : nullptr;
+    return launch_dn<false>(pool, d, idx, wgt, nullptr, H, Y, y_f32, batch, s, ys);
 }
 
 // The block: three launches (KQ_MOE_PATH_ONE: the one-launch kernel). With
@@ -2854,7 +2911,7 @@ hipError_t launch_moe_block(const uint8_t* pool, const kq_moe_desc& d, const voi
         e = launch_router_t<false>(R, r_f32, X, x_f32, batch, d, xh, ws, idx, wgt, s);
         if (e != hipSuccess) return e;
         const GuTopk tk{reinterpret_cast<const float*>(w + L.lg), idx, wgt, plan};
-        e = launch_gu_part(pool, d, xin, H, batch, tk, s);
+        e = launch_gu_part<false>(pool, d, xin, H, batch, tk, s);
     } else {
         e = launch_router(R, r_f32, X, x_f32, batch, d, xh, ws, idx, wgt, s);
         if (e != hipSuccess) return e;

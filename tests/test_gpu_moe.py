@@ -199,6 +199,34 @@ def test_gate_up_and_down_vs_oracle(gpu, pool16, batch):
     assert_close(to_f64(b.y), Yref, atol=1e-4, rtol=1e-4, what="down+combine")
 
 
+@pytest.mark.parametrize("tk,batch,kind", [(4, 2, "same"), (8, 16, "same"), (8, 16, "mixed"),
+                                           (4, 7, "mixed"), (4, 16, "one")])
+def test_standalone_repeated_experts(gpu, slot_pools, tk, batch, kind):
+    """A caller's routing that names experts more than once a token: plan
+    entries with up to 128 slots, cut for the partitioned kernels; down with
+    the workspace and without (LDS combine), against the oracle."""
+    d, host, pool = slot_pools[(256, 8)]
+    d = kq.MoEDesc(**{**d.as_dict(), "top_k": tk})
+    rng = np.random.default_rng(tk * batch)
+    idx = {"same": np.full((batch, tk), 200), "mixed": rng.integers(0, 3, (batch, tk)),
+           "one": np.stack([rng.permutation(256)[:tk] for _ in range(batch)])}[kind].astype(np.uint32)
+    if kind == "one":
+        idx[3] = 9
+    wgt = rng.dirichlet(np.ones(tk), batch).astype(np.float32)
+    X = gen.f16_bits(rng.normal(0, 1, (batch, 256)))
+    b = Block(gpu, d, batch)
+    idx_d, wgt_d = dev(idx, gpu), torch.from_numpy(wgt).to(gpu)
+    kq.moe_gate_up_swiglu(pool, d, idx_d, dev(X, gpu), b.H, b.ws, b.wsb, batch=batch)
+    torch.cuda.synchronize()
+    assert_close(to_f64(b.H), oracle.moe_gate_up(host, odesc(d), idx, X, oracle.F16, batch), what="h")
+    Yref = oracle.moe_down(host, odesc(d), idx, wgt.astype(np.float64), host_bits(b.H, np.uint16), batch)
+    for ws, wsb in ((b.ws, b.wsb), (None, 0), (b.ws, 256)):
+        b.y.fill_(float("nan"))
+        kq.moe_down_combine(pool, d, idx_d, wgt_d, b.H, b.y, ws, wsb, batch=batch)
+        torch.cuda.synchronize()
+        assert_close(to_f64(b.y), Yref, atol=1e-4, rtol=1e-4, what=f"down {wsb}")
+
+
 def test_duplicate_and_shared_experts(gpu, pool16):
     """Slots that select the same expert (within and across tokens) read its
     rows once and still land in their own h / y slots."""
