@@ -62,8 +62,11 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     kq::Int4Cfg mcfg = forced ? *forced : kq::int4_mfma_default(M, K, batch);
     const bool valu_ok = kq::int4_valu_supported(K, batch, vcfg);
     // the matrix-core path reads a span's separate scales / biases as one
-    // 4- or 8-byte word each
-    const bool meta_aligned = inter || (aligned(S, 8) && aligned(B, 8));
+    // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
+    // last two spans: with an odd number of spans that word would end past the
+    // array, and the range check would zero it
+    const bool meta_aligned =
+        inter || (aligned(S, 8) && aligned(B, 8) && !(G == 128 && (K / 128) % 2 != 0));
     const bool mfma_ok = meta_aligned && kq::int4_mfma_supported(M, K, G, batch, mcfg);
     // Crossover, in batch-1 vector passes: a vector pass takes up to 4 tokens
     // (int4_valu_cost), a matrix-core pass all of them at ~1.2 (29.3-30.3 us
@@ -85,6 +88,17 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
             const bool faster = mp * kq::int4_mfma_us(M, K, G, batch, mcfg) < kq::int4_valu_us(M, K, G, batch);
             path = fewer_passes && faster ? KQ_PATH_MFMA : KQ_PATH_VALU;
         }
+        // the skinny matrix-core kernels, any K of at least 256 (shapes that
+        // neither path takes stay refused): against the
+        // matrix cores' choice by size (int4_skinny_beats_mfma), against the
+        // vector path by duration (4096x4096: vector 5.4, skinny 6.0 us at 3
+        // tokens, 6.4 and 6.0 at 4, 10.0 and 6.1 at 5)
+        kq::skinny::Plan sp;
+        if (batch > 1 && (valu_ok || mfma_ok) && kq::int4_skinny_plan(M, K, G, batch, inter, sp) &&
+            (path == KQ_PATH_MFMA
+                 ? kq::int4_skinny_beats_mfma(sp, M, G, batch, inter)
+                 : !valu_ok || kq::skinny_us(sp, batch) < kq::int4_valu_pass_us(M, K, G, batch)))
+            return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
     }
     if (path == KQ_PATH_VALU) {
         if (!valu_ok) return KQ_EUNSUPPORTED;

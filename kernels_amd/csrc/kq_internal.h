@@ -22,8 +22,10 @@ Int4Cfg int4_valu_default(uint32_t M, uint32_t K, uint32_t batch);
 size_t int4_valu_lds_bytes(uint32_t K, uint32_t batch);
 // `batch` tokens on the vector path in batch-1-pass units x 100 (AUTO's crossover).
 uint32_t int4_valu_cost(uint32_t M, uint32_t K, uint32_t batch);
-// Modelled duration (us) of `batch` tokens on the vector path (AUTO's crossover).
+// Modelled duration (us) of `batch` tokens on the vector path (AUTO's
+// crossovers, with int4_mfma and with the skinny kernels).
 double int4_valu_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch);
+double int4_valu_pass_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch);
 
 // gsel (device pointer, may be null): the kernel reads the matrix index
 // gsel[0] and moves W, S and B by gsel[0] * gstride bytes -- one matrix of a
@@ -44,6 +46,28 @@ Int4Cfg int4_mfma_default(uint32_t M, uint32_t K, uint32_t batch);
 uint32_t int4_mfma_tokens_per_pass(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg);
 // Modelled duration (us) of one matrix-core pass (AUTO's crossover).
 double int4_mfma_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg);
+
+// Skinny matrix-core kernels (kq_skinny.hip), 1-16 tokens in one pass: the
+// launch plan (false: a shape they don't take), its modelled duration, and
+// whether it beats int4_mfma.
+namespace skinny {
+struct Plan {
+    uint32_t T, P, Q, J, NP, rounds, tiles_wg, nwg;
+    size_t part_lds, x_lds;  // the K-part sums, the waves' x stages
+};
+}  // namespace skinny
+bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl);
+double skinny_us(const skinny::Plan& pl, uint32_t batch);
+bool int4_skinny_beats_mfma(const skinny::Plan& pl, uint32_t M, uint32_t G, uint32_t batch, bool inter);
+hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
+                              bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
+                              uint32_t K, uint32_t G, uint32_t batch, const skinny::Plan& pl,
+                              hipStream_t s);
+bool vq_skinny_plan(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch,
+                    skinny::Plan& pl);
+hipError_t launch_vq_skinny(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
+                            void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
+                            uint32_t scale_group, uint32_t batch, const skinny::Plan& pl, hipStream_t s);
 
 // Debug scalar path: one thread per (row, token), plain chunk loop (v0).
 hipError_t launch_int4_scalar(const uint32_t* W, const uint16_t* S, const uint16_t* B,

@@ -500,6 +500,22 @@ hipError_t qgo_nb(const QArgs& a, const QPlan& pl, hipStream_t s) {
 
 }  // namespace
 
+// Which calls the skinny matrix-core kernels take (where they can). A pass here
+// carries up to 4 tokens and spreads rows over every CU; there all tokens go in
+// one pass, 16 rows a workgroup. Measured, passes / skinny (codebook per 256
+// rows, a scale per row): 5+ tokens always -- 9 tokens 14336x4096 36.4 / 13.8
+// us, 300x28672 37.2 / 20.8; 3 tokens (two passes) 4096x4096 9.3 / 5.5,
+// 1024x4096 7.7 / 5.3, but 300x28672 13.5 / 15.0; 4 tokens (one pass) 4096x4096
+// 6.7 / 5.6, 700x608 4.9 / 3.7, but 1024x4096 5.1 / 5.2; 2 tokens 28672x512 10.5
+// / 5.7, but 4096x4096 5.3 / 5.5.
+bool vq_skinny_pays(uint32_t M, uint32_t K, uint32_t batch) {
+    const uint32_t cu = cu_count(), ntiles = (M + 15) / 16;
+    if (batch >= 5) return true;
+    if (batch == 4) return ntiles * 2 >= cu || K <= 2048;
+    if (batch == 3) return ntiles * 8 >= cu || K <= 8192;
+    return batch == 2 && ntiles > cu && K <= 2048;
+}
+
 bool vq_supported(uint32_t M, uint32_t K, uint32_t rows_per_cb) {
     QPlan pl;
     return make_qplan(M, K, 1, rows_per_cb, pl);
@@ -508,6 +524,9 @@ bool vq_supported(uint32_t M, uint32_t K, uint32_t rows_per_cb) {
 hipError_t launch_vq(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
                      void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                      uint32_t scale_group, uint32_t batch, hipStream_t s) {
+    skinny::Plan sp;
+    if (vq_skinny_pays(M, K, batch) && vq_skinny_plan(M, K, rows_per_cb, scale_group, batch, sp))
+        return launch_vq_skinny(IDX, C, S, X, Y, y_f32, M, K, rows_per_cb, scale_group, batch, sp, s);
     uint32_t sgs = 0;
     while ((1u << sgs) < scale_group) ++sgs;
     const bool per_row = scale_group == K;

@@ -48,3 +48,51 @@ def test_config2_skinny(problem, batch, path):
     what = f"{M}x{K} batch {batch} path {path}"
     assert_close(got, ref[:batch], what=what)
     assert inf_rel(got, ref[:batch]) < 2e-3, what
+
+
+# The skinny kernels' edges, against the vector path's oracle: K = one pair of
+# spans, a last pair that overlaps, several rounds, partial tiles and last
+# workgroups, one K part and many, both x forms (8 / 9 tokens), every layout.
+# 2e-3 + 1e-4 |y|: float32 sums of products that carry up to 1024 + q are 1.3e-5
+# of y's size (up to ~30) off, five times that at the worst of 1e5 values; the
+# small shapes that another path takes included.
+SKINNY = [(1, 256, 64), (17, 288, 32), (300, 608, 32), (4097, 320, 64), (9000, 256, 128),
+          (5003, 2848, 32), (2880, 5056, 64), (6144, 1152, 128)]
+
+
+@pytest.mark.parametrize("layout,sb", [("sb", kq.F16), ("sb", kq.BF16), ("split", kq.F16), ("split", kq.BF16)])
+@pytest.mark.parametrize("M,K,G", SKINNY)
+def test_skinny_edges(gpu, M, K, G, layout, sb):
+    for batch in (5, 8, 9, 16):
+        p = gen.int4_problem(M, K, G, batch=batch, seed=M + K + batch)
+        if sb == kq.BF16:
+            f = lambda a: gen.bf16_bits(a.view(np.float16).astype(np.float32))  # noqa: E731
+            p = dict(p, S=f(p["S"]), B=f(p["B"]), SB=f(p["SB"]))
+        S, B = (p["SB"], None) if layout == "sb" else (p["S"], p["B"])
+        y = torch.full((batch, M), float("nan"), dtype=torch.float32, device=gpu)
+        kq.int4_gemv(dev(p["W"], gpu), dev(S, gpu), dev(p["X"], gpu), y, kq.GemvParams(M, K, G),
+                     B=None if B is None else dev(B, gpu), batch=batch, sb_dtype=sb)
+        torch.cuda.synchronize()
+        ref = oracle.int4_gemv(p["W"], S, B, p["X"], M, K, G, layout == "sb",
+                               oracle.BF16 if sb == kq.BF16 else oracle.F16)
+        assert_close(to_f64(y), ref, atol=2e-3, rtol=1e-4, what=f"{M}x{K} g{G} {layout} b{batch}")
+
+
+# The same for codebook weights: codebooks that end inside a tile or are
+# smaller than a workgroup's share (the passes), shares widened to divide one,
+# scale groups of every form.
+SKINNY_VQ = [(1, 256, 1, 256), (300, 288, 256, 288), (4100, 512, 256, 32), (700, 608, 16, 608),
+             (5000, 1024, 256, 64), (3000, 2048, 7, 2048), (9000, 256, 256, 128),
+             (2000, 5120, 2000, 512), (2900, 1088, 256, 32)]
+
+
+@pytest.mark.parametrize("M,K,rpc,sg", SKINNY_VQ)
+def test_skinny_vq_edges(gpu, M, K, rpc, sg):
+    for batch in (3, 5, 8, 9, 16):
+        p = gen.vq_problem(M, K, rows_per_cb=rpc, scale_group=sg, batch=batch, seed=M + K + batch)
+        y = torch.full((batch, M), float("nan"), dtype=torch.float32, device=gpu)
+        kq.vq_gemv(dev(p["IDX"], gpu), dev(p["C"], gpu), dev(p["S"], gpu), dev(p["X"], gpu), y,
+                   kq.VQParams(M, K, rpc, sg), batch=batch)
+        torch.cuda.synchronize()
+        ref = oracle.vq_gemv(p["IDX"], p["C"], p["S"], p["X"], M, K, rpc, sg)
+        assert_close(to_f64(y), ref, atol=2e-5, rtol=1e-6, what=f"vq {M}x{K} cb{rpc} sg{sg} b{batch}")
