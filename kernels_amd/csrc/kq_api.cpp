@@ -61,13 +61,17 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     kq::Int4Cfg vcfg = forced ? *forced : kq::int4_valu_default(M, K, batch);
     kq::Int4Cfg mcfg = forced ? *forced : kq::int4_mfma_default(M, K, batch);
     const bool valu_ok = kq::int4_valu_supported(K, batch, vcfg);
+    // one token is the vector path's (its cost is the crossover's unit, 100
+    // against 120); the other paths' plans are not looked at (1.5 us of host
+    // time a call)
+    if (path == KQ_PATH_AUTO && batch == 1 && valu_ok) path = KQ_PATH_VALU;
     // the matrix-core path reads a span's separate scales / biases as one
     // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
     // last two spans: with an odd number of spans that word would end past the
     // array, and the range check would zero it
     const bool meta_aligned =
         inter || (aligned(S, 8) && aligned(B, 8) && !(G == 128 && (K / 128) % 2 != 0));
-    const bool mfma_ok = meta_aligned && kq::int4_mfma_supported(M, K, G, batch, mcfg);
+    const bool mfma_ok = path != KQ_PATH_VALU && meta_aligned && kq::int4_mfma_supported(M, K, G, batch, mcfg);
     // Crossover, in batch-1 vector passes: a vector pass takes up to 4 tokens
     // (int4_valu_cost), a matrix-core pass all of them at ~1.2 (29.3-30.3 us
     // against 24.9 us at 28672 x 8192; 64-byte row pieces per load instead of

@@ -120,10 +120,17 @@ def _ptr(t):
     return t.data_ptr()
 
 
+_current = None  # (raw stream of a device, current device): torch's own, without a Stream object
+
+
 def _stream(stream):
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        global _current
+        if _current is None:
+            import torch
+            torch.cuda.init()
+            _current = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+        return _current[0](_current[1]())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -134,9 +141,15 @@ def _check(st, where):
         raise KQError(st, where)
 
 
+_dtypes = None
+
+
 def _dt(t):
-    import torch
-    return {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}[t.dtype]
+    global _dtypes
+    if _dtypes is None:
+        import torch
+        _dtypes = {torch.float16: F16, torch.bfloat16: BF16, torch.float32: F32}
+    return _dtypes[t.dtype]
 
 
 # ---------------------------------------------------------------------------
