@@ -183,7 +183,8 @@ kq_status kq_vq_gemv(const uint8_t* IDX, const uint16_t* C, const uint16_t* S,
  * (else KQ_EUNSUPPORTED).
  * ws: kq_vq_quantize_workspace_size bytes, 256-byte aligned (the scales,
  * the sample, the centroids and their sums); 0 means invalid arguments.
- * Launches: 3 + 2 * iters.
+ * Launches: 4 + 2 * iters (3 + 2 * iters where IDX and the sample have no
+ * room for the cells' candidate lists). IDX is scratch memory meanwhile.
  *
  * Replaces: quantize_matrix / _kmeans vq-gemv/quant/pq_quantize.py:28-83
  *   (reference defaults: iters 25, sample 200000, scale_group 32,
@@ -271,6 +272,8 @@ kq_status kq_moe_gate_up_swiglu(const uint8_t* pool, const kq_moe_desc* d,
 
 /* Y[b][m] = sum_k wgt[b][k] * (down_e(H[b][k])[m] + BId[m]), e = idx[b][k],
  * summed in k order. Y: [batch][hidden] of y_dtype (KQ_F32 or KQ_F16).
+ * A workspace (optional) may take the per-slot products (6 or more tokens), so
+ * it must not be in use by work on another stream.
  * Replaces: fused_down_combine moe-fused/src/kernels.metal:224-265
  *   (encoded at moe-fused/src/main.mm:196-204). */
 kq_status kq_moe_down_combine(const uint8_t* pool, const kq_moe_desc* d,

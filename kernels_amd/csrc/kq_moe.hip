@@ -32,10 +32,12 @@
 //      expert with only that expert's activations in LDS; down writes
 //      per-slot products to the workspace and a small moe_combine_k launch
 //      sums them in slot order (4 launches in all);
-//    - per tile (moe_gate_up_k, moe_down_k): the standalone entry points
-//      past the streaming limits (they take no workspace): a grid of
-//      (16-row tile, expert) or 8-output-row workgroups that issue all of
-//      their loads in one round trip.
+//      The standalone entry points run them too, on the caller's idx (down
+//      where it has a workspace).
+//    - per tile (moe_gate_up_k, moe_down_k): shapes past the LDS limits and
+//      a standalone down without a workspace: a grid of (16-row tile,
+//      expert) or 8-output-row workgroups that issue all of their loads in
+//      one round trip.
 //    Every form reads each selected expert's rows once per call for all
 //    token slots that chose it; a half-wave owns one row of a pair (gate /
 //    up, or two down rows; K = 2880 = 90 chunks -> 3 per lane), so SwiGLU
