@@ -69,9 +69,15 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
     // last two spans: with an odd number of spans that word would end past the
     // array, and the range check would zero it
-    const bool meta_aligned =
-        inter || (aligned(S, 8) && aligned(B, 8) && !(G == 128 && (K / 128) % 2 != 0));
-    const bool mfma_ok = path != KQ_PATH_VALU && meta_aligned && kq::int4_mfma_supported(M, K, G, batch, mcfg);
+    const bool mfma_shape = path != KQ_PATH_VALU && (inter || (aligned(S, 8) && aligned(B, 8))) &&
+                            kq::int4_mfma_supported(M, K, G, batch, mcfg);
+    const bool mfma_ok = mfma_shape && (inter || G != 128 || (K / 128) % 2 == 0);
+    // ... those go to the skinny kernels where the matrix cores are asked for, or
+    // the only path that takes K
+    kq::skinny::Plan sp;
+    if (mfma_shape && !mfma_ok && (path == KQ_PATH_MFMA || (path == KQ_PATH_AUTO && !valu_ok)) &&
+        kq::int4_skinny_plan(M, K, G, batch, inter, sp))
+        return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
     // Crossover, in batch-1 vector passes: a vector pass takes up to 4 tokens
     // (int4_valu_cost), a matrix-core pass all of them at ~1.2 (29.3-30.3 us
     // against 24.9 us at 28672 x 8192; 64-byte row pieces per load instead of
@@ -97,7 +103,6 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
         // matrix cores' choice by size (int4_skinny_beats_mfma), against the
         // vector path by duration (4096x4096: vector 5.4, skinny 6.0 us at 3
         // tokens, 6.4 and 6.0 at 4, 10.0 and 6.1 at 5)
-        kq::skinny::Plan sp;
         if (batch > 1 && (valu_ok || mfma_ok) && kq::int4_skinny_plan(M, K, G, batch, inter, sp) &&
             (path == KQ_PATH_MFMA
                  ? kq::int4_skinny_beats_mfma(sp, M, G, batch, inter)

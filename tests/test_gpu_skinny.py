@@ -96,3 +96,19 @@ def test_skinny_vq_edges(gpu, M, K, rpc, sg):
         torch.cuda.synchronize()
         ref = oracle.vq_gemv(p["IDX"], p["C"], p["S"], p["X"], M, K, rpc, sg)
         assert_close(to_f64(y), ref, atol=2e-5, rtol=1e-6, what=f"vq {M}x{K} cb{rpc} sg{sg} b{batch}")
+
+
+# Separate scales of 128-wide groups with an odd number of spans, which
+# int4_mfma does not take: the matrix-core path asked for by name, and a K that
+# the vector path's LDS does not hold. 1e-5 of the largest value: float32 sums of
+# products that carry 64 + q measure about 1e-6.
+@pytest.mark.parametrize("M,K,path", [(300, 1152, kq.PATH_MFMA), (17, 131200, kq.PATH_AUTO)])
+def test_odd_spans_split_g128(gpu, M, K, path):
+    for batch in (1, 5, 16):
+        p = gen.int4_problem(M, K, 128, batch=batch, seed=K + batch)
+        y = torch.full((batch, M), float("nan"), dtype=torch.float32, device=gpu)
+        kq.int4_gemv(dev(p["W"], gpu), dev(p["S"], gpu), dev(p["X"], gpu), y, kq.GemvParams(M, K, 128),
+                     B=dev(p["B"], gpu), batch=batch, path=path)
+        torch.cuda.synchronize()
+        ref = oracle.int4_gemv(p["W"], p["S"], p["B"], p["X"], M, K, 128, False, oracle.F16)
+        assert inf_rel(to_f64(y), ref) < 1e-5, f"{M}x{K} b{batch}"
