@@ -106,7 +106,7 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
         if (batch > 1 && (valu_ok || mfma_ok) && kq::int4_skinny_plan(M, K, G, batch, inter, sp) &&
             (path == KQ_PATH_MFMA
                  ? kq::int4_skinny_beats_mfma(sp, M, G, batch, inter)
-                 : !valu_ok || kq::skinny_us(sp, batch) < kq::int4_valu_pass_us(M, K, G, batch)))
+                 : !valu_ok || kq::int4_skinny_us(sp, batch) < kq::int4_valu_pass_us(M, K, G, batch)))
             return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
     }
     if (path == KQ_PATH_VALU) {

@@ -57,7 +57,7 @@ struct Plan {
 };
 }  // namespace skinny
 bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl);
-double skinny_us(const skinny::Plan& pl, uint32_t batch);
+double int4_skinny_us(const skinny::Plan& pl, uint32_t batch);
 bool int4_skinny_beats_mfma(const skinny::Plan& pl, uint32_t M, uint32_t G, uint32_t batch, bool inter);
 hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                               bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
@@ -65,6 +65,10 @@ hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16
                               hipStream_t s);
 bool vq_skinny_plan(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch,
                     skinny::Plan& pl);
+double vq_skinny_us(const skinny::Plan& pl, uint32_t K, uint32_t scale_group, uint32_t batch);
+bool vq_skinny_usable(uint32_t K, uint32_t scale_group);  // as loaded on this device
+// Whether a call takes them (kq_vq.hip), were they usable.
+bool vq_takes_skinny(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch);
 hipError_t launch_vq_skinny(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
                             void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                             uint32_t scale_group, uint32_t batch, const skinny::Plan& pl, hipStream_t s);

@@ -15,12 +15,11 @@ namespace {
 
 constexpr size_t kLdsMax = 160 * 1024;
 
-// Modelled duration: a launch with its first loads and the K-part sums, then
-// a wave's steps at 8 waves a CU (a step: T tiles and the x of 256 k) -- 1.25 /
-// 2.0 / 4.3 us at T = 1 / 2 / 4 up to 8 tokens, 2.05 / 2.7 / 4.9 us above --
-// and 1 us a further round (fitted: 1024x4096 .. 8192x28672, most within 10%).
-// Fewer tiles a step pay for x again, more leave fewer waves to hide a step's
-// serial chain.
+// What orders a shape's plans: a launch with its first loads and the K-part sums,
+// then a wave's steps at 8 waves a CU (a step: T tiles and the x of 256 k) --
+// 1.25 / 2.0 / 4.3 us at T = 1 / 2 / 4 up to 8 tokens, 2.05 / 2.7 / 4.9 us above
+// -- and 1 us a further round. Fewer tiles a step pay for x again, more leave
+// fewer waves to hide a step's serial chain.
 double plan_us(const skinny::Plan& pl, uint32_t batch) {
     const int t = pl.T == 1 ? 0 : pl.T == 2 ? 1 : 2;
     static constexpr double kStep[2][3] = {{1.25, 2.0, 4.3}, {2.05, 2.7, 4.9}};
@@ -107,7 +106,21 @@ int vq_gm(uint32_t K, uint32_t scale_group) {
 
 }  // namespace
 
-double skinny_us(const skinny::Plan& pl, uint32_t batch) { return plan_us(pl, batch); }
+// Modelled duration of a plan, which the choice between paths goes by: a launch,
+// then a wave's steps, one part fixed and one that grows with the waves a CU and
+// a little with the CUs in use. form: a step's cost by scale layout (fitted
+// together over both formats: 250-28672 rows, K 512-28672, 3000 calls, nineteen in
+// twenty within 15%).
+static double skinny_us(const skinny::Plan& pl, uint32_t batch, double form) {
+    static constexpr double kStep[2][3] = {{0.0, 0.1, 0.0}, {0.2, 1.6, 4.74}},
+                            kWaves[2][3] = {{1.37, 2.14, 4.06}, {1.7, 1.25, 0.0}};
+    const int t = pl.T == 1 ? 0 : pl.T == 2 ? 1 : 2, b = batch > 8;
+    const double fill = pl.P * pl.Q / 8.0 * (0.8 + 0.2 * pl.nwg / cu_count());
+    return 3.2 + (double)pl.rounds * pl.J * (kStep[b][t] + kWaves[b][t] * fill) * form;
+}
+
+// (the choice against the vector path still goes by plan_us)
+double int4_skinny_us(const skinny::Plan& pl, uint32_t batch) { return plan_us(pl, batch); }
 
 bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl) {
     if (batch < 1 || batch > 16 || !(G == 32 || G == 64 || G == 128) || K % G) return false;
@@ -154,8 +167,15 @@ bool vq_skinny_plan(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale
     if (batch < 1 || batch > 16) return false;
     const int gm = vq_gm(K, scale_group);
     const uint32_t per = vq_share(M, rows_per_cb);
-    return per != 0 && make_plan(M, K, batch, gm == 32 ? 2 : 4, per, kCbLds, pl) && skinny_vq_usable(gm);
+    return per != 0 && make_plan(M, K, batch, gm == 32 ? 2 : 4, per, kCbLds, pl);
 }
+
+double vq_skinny_us(const skinny::Plan& pl, uint32_t K, uint32_t scale_group, uint32_t batch) {
+    const int gm = vq_gm(K, scale_group);
+    return skinny_us(pl, batch, gm == 32 ? 1.1 : gm == 64 ? 1.02 : 1.0);
+}
+
+bool vq_skinny_usable(uint32_t K, uint32_t scale_group) { return skinny_vq_usable(vq_gm(K, scale_group)); }
 
 hipError_t launch_vq_skinny(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
                             void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,

@@ -498,22 +498,72 @@ hipError_t qgo_nb(const QArgs& a, const QPlan& pl, hipStream_t s) {
     return pl.R == 2 ? qgo<NB, 2, 1>(a, pl, s) : qgo<NB, 1, 1>(a, pl, s);
 }
 
+// The passes of `batch` tokens: 4 tokens each, then 2, then 1 (fewer where x
+// does not fit LDS), `times` of them on one plan.
+struct QPass {
+    uint32_t nb, times;
+    QPlan pl;
+};
+uint32_t make_qpasses(uint32_t M, uint32_t K, uint32_t batch, uint32_t rpc, QPass (&out)[3]) {
+    uint32_t n = 0;
+    for (uint32_t nb : {4u, 2u, 1u}) {
+        if (batch < nb || !make_qplan(M, K, nb, rpc, out[n].pl)) continue;
+        out[n].nb = nb;
+        out[n++].times = batch / nb;
+        batch %= nb;
+    }
+    return batch ? 0 : n;
+}
+
+// Their modelled duration: per pass of 1 / 2 / 4 tokens a launch with its ramp,
+// a CU's 1 KiB index pieces, the x that each of its waves stages (2048 k) and a
+// wave's own pieces one after another (fitted: 250-28672 rows, K 512-28672,
+// codebooks of 1 row to all, 1600 calls, nineteen in twenty within 12%).
+double passes_us(const QPass* ps, uint32_t n, uint32_t K) {
+    double us = 0.0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const QPlan& pl = ps[i].pl;
+        const uint32_t waves = pl.P * pl.Q, j = ps[i].nb == 4 ? 2 : ps[i].nb - 1;
+        static constexpr double kFix[3] = {2.8, 3.15, 3.4}, kPiece[3] = {0.028, 0.057, 0.074},
+                                kStage[3] = {0.53, 1.55, 2.05}, kChain[3] = {0.28, 0.11, 0.29};
+        const double wave_pieces = pl.nreal * pl.R;
+        us += ps[i].times * (kFix[j] + kPiece[j] * wave_pieces * waves +
+                             kStage[j] * ((K + 2047) / 2048) / (waves < 8 ? waves : 8) +
+                             kChain[j] * wave_pieces);
+    }
+    return us;
+}
+
 }  // namespace
 
-// Which calls the skinny matrix-core kernels take (where they can). A pass here
-// carries up to 4 tokens and spreads rows over every CU; there all tokens go in
-// one pass, 16 rows a workgroup. Measured, passes / skinny (codebook per 256
-// rows, a scale per row): 5+ tokens always -- 9 tokens 14336x4096 36.4 / 13.8
-// us, 300x28672 37.2 / 20.8; 3 tokens (two passes) 4096x4096 9.3 / 5.5,
-// 1024x4096 7.7 / 5.3, but 300x28672 13.5 / 15.0; 4 tokens (one pass) 4096x4096
-// 6.7 / 5.6, 700x608 4.9 / 3.7, but 1024x4096 5.1 / 5.2; 2 tokens 28672x512 10.5
-// / 5.7, but 4096x4096 5.3 / 5.5.
-bool vq_skinny_pays(uint32_t M, uint32_t K, uint32_t batch) {
+// Which calls the skinny matrix-core kernels take (where they can): one pass
+// carries all tokens there, 16-row tiles a workgroup, where a pass here carries
+// up to 4 and spreads single rows over every CU. Up to 4 tokens the sizes below
+// limit it: 3 tokens (two passes) 4096x4096 passes 9.3 / skinny 5.5 us, but
+// 300x28672 13.5 / 15.0; 4 tokens (one pass) 4096x4096 6.7 / 5.6, 700x608 4.9 /
+// 3.7, but 1940x3488 5.3 / 6.1; 2 tokens 28672x512 10.5 / 5.7, but 4096x4096 5.3 /
+// 5.5. Then the modelled durations decide: codebook blocks whose tiles divide
+// badly leave few workgroups there (11008x4096, a codebook per 1376 rows, 4
+// tokens: 12.4 us in passes, 67 on 16 workgroups; 28672x8192, per 4112, 8 tokens:
+// 99 / 719), while 9 tokens of 14336x4096 (per 256) take 36.4 / 13.8 and 5 of
+// 300x28672 (one codebook) 20.2 / 15.2.
+namespace {
+bool skinny_pays(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch,
+                 const QPass* ps, uint32_t n, skinny::Plan& sp) {
     const uint32_t cu = cu_count(), ntiles = (M + 15) / 16;
-    if (batch >= 5) return true;
-    if (batch == 4) return ntiles * 2 >= cu || K <= 2048;
-    if (batch == 3) return ntiles * 8 >= cu || K <= 8192;
-    return batch == 2 && ntiles > cu && K <= 2048;
+    if (batch < 2 || (batch == 2 && (ntiles <= cu || K > 2048)) ||
+        (batch == 3 && ntiles * 8 < cu && K > 8192) || (batch == 4 && ntiles * 2 < cu && K > 2048))
+        return false;
+    return vq_skinny_plan(M, K, rows_per_cb, scale_group, batch, sp) &&
+           0.95 * vq_skinny_us(sp, K, scale_group, batch) < passes_us(ps, n, K);
+}
+}  // namespace
+
+bool vq_takes_skinny(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch) {
+    QPass ps[3];
+    skinny::Plan sp;
+    const uint32_t n = make_qpasses(M, K, batch, rows_per_cb, ps);
+    return n != 0 && skinny_pays(M, K, rows_per_cb, scale_group, batch, ps, n, sp);
 }
 
 bool vq_supported(uint32_t M, uint32_t K, uint32_t rows_per_cb) {
@@ -524,20 +574,19 @@ bool vq_supported(uint32_t M, uint32_t K, uint32_t rows_per_cb) {
 hipError_t launch_vq(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
                      void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                      uint32_t scale_group, uint32_t batch, hipStream_t s) {
+    QPass ps[3];
+    const uint32_t n = make_qpasses(M, K, batch, rows_per_cb, ps);
+    if (n == 0) return hipErrorInvalidValue;
     skinny::Plan sp;
-    if (vq_skinny_pays(M, K, batch) && vq_skinny_plan(M, K, rows_per_cb, scale_group, batch, sp))
+    if (skinny_pays(M, K, rows_per_cb, scale_group, batch, ps, n, sp) && vq_skinny_usable(K, scale_group))
         return launch_vq_skinny(IDX, C, S, X, Y, y_f32, M, K, rows_per_cb, scale_group, batch, sp, s);
     uint32_t sgs = 0;
     while ((1u << sgs) < scale_group) ++sgs;
     const bool per_row = scale_group == K;
     const size_t ysz = y_f32 ? 4 : 2;
-    for (uint32_t t0 = 0; t0 < batch;) {
-        uint32_t nb = batch - t0 >= 4 ? 4 : batch - t0 >= 2 ? 2 : 1;
-        QPlan pl;
-        while (!make_qplan(M, K, nb, rows_per_cb, pl)) {
-            if (nb == 1) return hipErrorInvalidValue;
-            nb /= 2;
-        }
+    for (uint32_t t0 = 0, i = 0; t0 < batch; i += --ps[i].times == 0) {
+        const QPlan& pl = ps[i].pl;
+        const uint32_t nb = ps[i].nb;
         QArgs a;
         a.IDX = IDX;
         a.C = C;

@@ -112,3 +112,17 @@ def test_odd_spans_split_g128(gpu, M, K, path):
         torch.cuda.synchronize()
         ref = oracle.int4_gemv(p["W"], p["S"], p["B"], p["X"], M, K, 128, False, oracle.F16)
         assert inf_rel(to_f64(y), ref) < 1e-5, f"{M}x{K} b{batch}"
+
+
+# Codebook blocks of an odd tile count: the skinny kernels with a workgroup a
+# block, or the passes, whichever the route gives.
+@pytest.mark.parametrize("M,K,rpc,sg", [(5120, 512, 1264, 512), (2768, 1056, 592, 32), (4128, 288, 1376, 288)])
+def test_vq_uneven_codebook_blocks(gpu, M, K, rpc, sg):
+    for batch in (3, 8, 16):
+        p = gen.vq_problem(M, K, rows_per_cb=rpc, scale_group=sg, batch=batch, seed=M + K + batch)
+        y = torch.full((batch, M), float("nan"), dtype=torch.float32, device=gpu)
+        kq.vq_gemv(dev(p["IDX"], gpu), dev(p["C"], gpu), dev(p["S"], gpu), dev(p["X"], gpu), y,
+                   kq.VQParams(M, K, rpc, sg), batch=batch)
+        torch.cuda.synchronize()
+        ref = oracle.vq_gemv(p["IDX"], p["C"], p["S"], p["X"], M, K, rpc, sg)
+        assert_close(to_f64(y), ref, atol=2e-5, rtol=1e-6, what=f"vq {M}x{K} cb{rpc} sg{sg} b{batch}")
