@@ -58,9 +58,15 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     const auto* Bp = static_cast<const uint16_t*>(B);
     const bool yf = y_dtype == KQ_F32;
 
-    kq::Int4Cfg vcfg = forced ? *forced : kq::int4_valu_default(M, K, batch);
-    kq::Int4Cfg mcfg = forced ? *forced : kq::int4_mfma_default(M, K, batch);
-    const bool valu_ok = kq::int4_valu_supported(K, batch, vcfg);
+    // the plan of each path that the call may take, made once
+    const kq::Int4Cfg cfg = forced ? *forced : kq::Int4Cfg{0, 0};
+    kq::Int4Passes vp;
+    vp.n = 0;
+    bool valu_ok = false;
+    if (path == KQ_PATH_AUTO || path == KQ_PATH_VALU) {
+        vp = kq::int4_valu_passes(M, K, batch, cfg);
+        valu_ok = forced ? kq::int4_valu_supported(K, cfg) : vp.n != 0;
+    }
     // one token is the vector path's (its cost is the crossover's unit, 100
     // against 120); the other paths' plans are not looked at (1.5 us of host
     // time a call)
@@ -69,8 +75,10 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
     // last two spans: with an odd number of spans that word would end past the
     // array, and the range check would zero it
-    const bool mfma_shape = path != KQ_PATH_VALU && (inter || (aligned(S, 8) && aligned(B, 8))) &&
-                            kq::int4_mfma_supported(M, K, G, batch, mcfg);
+    kq::mfma::Plan mp;
+    const bool mfma_shape = (path == KQ_PATH_AUTO || path == KQ_PATH_MFMA) &&
+                            (inter || (aligned(S, 8) && aligned(B, 8))) &&
+                            kq::int4_mfma_plan(M, K, G, batch, cfg, mp);
     const bool mfma_ok = mfma_shape && (inter || G != 128 || (K / 128) % 2 == 0);
     // ... those go to the skinny kernels where the matrix cores are asked for, or
     // the only path that takes K
@@ -92,10 +100,8 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
         } else if (!valu_ok) {
             path = KQ_PATH_MFMA;
         } else {
-            const uint32_t tpp = kq::int4_mfma_tokens_per_pass(M, K, G, batch, mcfg);
-            const uint32_t mp = tpp ? (batch + tpp - 1) / tpp : 1000;
-            const bool fewer_passes = 120 * mp < kq::int4_valu_cost(M, K, batch);
-            const bool faster = mp * kq::int4_mfma_us(M, K, G, batch, mcfg) < kq::int4_valu_us(M, K, G, batch);
+            const bool fewer_passes = 120 < kq::int4_valu_cost(vp);
+            const bool faster = kq::int4_mfma_us(mp, batch) < kq::int4_valu_us(vp, M, K, G);
             path = fewer_passes && faster ? KQ_PATH_MFMA : KQ_PATH_VALU;
         }
         // the skinny matrix-core kernels, any K of at least 256 (shapes that
@@ -106,16 +112,16 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
         if (batch > 1 && (valu_ok || mfma_ok) && kq::int4_skinny_plan(M, K, G, batch, inter, sp) &&
             (path == KQ_PATH_MFMA
                  ? kq::int4_skinny_beats_mfma(sp, M, G, batch, inter)
-                 : !valu_ok || kq::int4_skinny_us(sp, batch) < kq::int4_valu_pass_us(M, K, G, batch)))
+                 : !valu_ok || kq::int4_skinny_us(sp, batch) < kq::int4_valu_pass_us(vp, M, K, G)))
             return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
     }
     if (path == KQ_PATH_VALU) {
         if (!valu_ok) return KQ_EUNSUPPORTED;
-        return hip_status(kq::launch_int4_valu(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, vcfg, s));
+        return hip_status(kq::launch_int4_valu(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, vp, s));
     }
     if (path == KQ_PATH_MFMA) {
         if (!mfma_ok) return KQ_EUNSUPPORTED;
-        return hip_status(kq::launch_int4_mfma(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, mcfg, s));
+        return hip_status(kq::launch_int4_mfma(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, mp, s));
     }
     if (path == KQ_PATH_SCALAR)
         return hip_status(kq::launch_int4_scalar(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, s));
@@ -497,8 +503,8 @@ kq_status kq_moe_block_unfused(const uint8_t* pool, const kq_moe_desc* d, const 
     if (!aligned(Y, y_dtype == KQ_F32 ? 4 : 2)) return KQ_EALIGN;
     if (!ws || ws_bytes < kq::moe_unfused_ws_bytes(*d)) return KQ_EWORKSPACE;
     if (!aligned(ws, 256)) return KQ_EALIGN;
-    if (!kq::int4_valu_supported(d->hidden, 1, kq::Int4Cfg{0, 0}) ||
-        !kq::int4_valu_supported(d->inter, 1, kq::Int4Cfg{0, 0}))
+    if (!kq::int4_valu_supported(d->hidden, kq::Int4Cfg{0, 0}) ||
+        !kq::int4_valu_supported(d->inter, kq::Int4Cfg{0, 0}))
         return KQ_EUNSUPPORTED;
     st = hip_status(kq::launch_moe_unfused(pool, *d, R, r_dtype == KQ_F32, X, x_dtype == KQ_F32,
                                            idx, wgt, xh, H, Y, y_dtype == KQ_F32, ws,

@@ -61,11 +61,6 @@ struct VArgs {
     uint64_t gstride;                 // bytes (one matrix of a pool, picked on the device)
 };
 
-struct VPlan {
-    uint32_t R, P, Q, J, rounds, groups_wg, nwg, nreal, nsteps, D, xw;
-    size_t lds;
-};
-
 template <int R, bool SB>
 struct VSlot;
 template <int R>
@@ -483,46 +478,54 @@ hipError_t vgo_nb(const VArgs& a, const VPlan& pl, bool sb, bool bf, hipStream_t
 
 }  // namespace
 
-Int4Cfg int4_valu_default(uint32_t, uint32_t, uint32_t) { return Int4Cfg{0, 0}; }
+// Passes of 4 tokens, then of the rest (of 2 or 1 where x does not fit LDS).
+Int4Passes int4_valu_passes(uint32_t M, uint32_t K, uint32_t batch, Int4Cfg cfg) {
+    Int4Passes ps;
+    ps.n = 0;
+    VPlan pl[kMaxNB + 1];
+    int known[kMaxNB + 1] = {};  // 1: planned, -1: no plan
+    while (batch) {
+        uint32_t nb = batch < kMaxNB ? batch : kMaxNB;
+        for (;; nb = nb > 2 ? 2 : 1) {
+            if (!known[nb]) known[nb] = make_vplan(M, K, nb, cfg, pl[nb]) ? 1 : -1;
+            if (known[nb] > 0) break;
+            if (nb == 1) {
+                ps.n = 0;
+                return ps;
+            }
+        }
+        if (ps.n && ps.p[ps.n - 1].nb == nb) ++ps.p[ps.n - 1].times;
+        else ps.p[ps.n++] = {nb, 1, pl[nb]};
+        batch -= nb;
+    }
+    return ps;
+}
 
-// Cost of `batch` tokens on the vector path in batch-1 passes: passes of 4,
-// then 3, 2 or 1 tokens (fewer where x does not fit LDS), a pass of n tokens
-// costing 1, 1.12, 1.37, 1.58 (x100) batch-1 passes -- measured at 28672 x
-// 8192 and 8192 x 28672 (24.9, 27.9, 34.1, 39.4 us at 1-4 tokens).
-uint32_t int4_valu_cost(uint32_t M, uint32_t K, uint32_t batch) {
+// A pass of 1-4 tokens costs 1, 1.12, 1.37, 1.58 (x100) batch-1 passes --
+// measured at 28672 x 8192 and 8192 x 28672 (24.9, 27.9, 34.1, 39.4 us).
+uint32_t int4_valu_cost(const Int4Passes& ps) {
     static constexpr uint32_t kPass[5] = {0, 100, 112, 137, 158};
     uint32_t cost = 0;
-    for (uint32_t t0 = 0; t0 < batch;) {
-        uint32_t nb = batch - t0 >= kMaxNB ? kMaxNB : batch - t0;
-        VPlan pl;
-        while (nb > 1 && !make_vplan(M, K, nb, Int4Cfg{0, 0}, pl)) nb = nb > 2 ? 2 : 1;
-        cost += kPass[nb];
-        t0 += nb;
-    }
+    for (uint32_t i = 0; i < ps.n; ++i) cost += ps.p[i].times * kPass[ps.p[i].nb];
     return cost;
 }
 
 // A batch-1 pass streams at ~5.3 TB/s after ~3 us of launch, ramp and tail
 // (fitted: 1024x4096 .. 28672x8192 measured at 2-4 tokens, within ~15%).
-double int4_valu_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch) {
+double int4_valu_us(const Int4Passes& ps, uint32_t M, uint32_t K, uint32_t G) {
     const double bytes = (double)M * K / 2 + (double)M * (K / G) * 4;
-    return int4_valu_cost(M, K, batch) / 100.0 * (3.0 + bytes / 5.3e6);
+    return int4_valu_cost(ps) / 100.0 * (3.0 + bytes / 5.3e6);
 }
 
 // The same, pass by pass, for small matrices: a pass of 1 / 2 / 3 / 4 tokens
 // takes 2.6 / 3.2 / 3.4 / 3.6 us and 0.165 / 0.205 / 0.28 / 0.34 us a MB, K in
 // whole 2048-k steps (fitted: 2048x2048 .. 20480x5120, most within 10%).
-double int4_valu_pass_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch) {
+double int4_valu_pass_us(const Int4Passes& ps, uint32_t M, uint32_t K, uint32_t G) {
     static constexpr double kFix[5] = {0, 2.6, 3.2, 3.4, 3.6}, kMb[5] = {0, 0.165, 0.205, 0.28, 0.34};
     const double kp = (double)((K + 2047) / 2048 * 2048), mb = (M * kp / 2 + M * (kp / G) * 4) / 1e6;
     double us = 0.0;
-    for (uint32_t t0 = 0; t0 < batch;) {
-        uint32_t nb = batch - t0 >= kMaxNB ? kMaxNB : batch - t0;
-        VPlan pl;
-        while (nb > 1 && !make_vplan(M, K, nb, Int4Cfg{0, 0}, pl)) nb = nb > 2 ? 2 : 1;
-        us += kFix[nb] + kMb[nb] * mb;
-        t0 += nb;
-    }
+    for (uint32_t i = 0; i < ps.n; ++i)
+        us += ps.p[i].times * (kFix[ps.p[i].nb] + kMb[ps.p[i].nb] * mb);
     return us;
 }
 
@@ -531,26 +534,22 @@ size_t int4_valu_lds_bytes(uint32_t K, uint32_t batch) {
     return vlds_x(batch < kMaxNB ? batch : kMaxNB, nchp);
 }
 
-bool int4_valu_supported(uint32_t K, uint32_t batch, Int4Cfg cfg) {
-    if (batch < 1 || batch > 16) return false;
+bool int4_valu_supported(uint32_t K, Int4Cfg cfg) {
     VPlan pl;
     return make_vplan(16, K, 1, cfg, pl);
 }
 
 hipError_t launch_int4_valu(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                             bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
-                            uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, hipStream_t s,
-                            const uint32_t* gsel, uint64_t gstride) {
+                            uint32_t K, uint32_t G, uint32_t batch, const Int4Passes& ps,
+                            hipStream_t s, const uint32_t* gsel, uint64_t gstride) {
     const size_t ysz = y_f32 ? 4 : 2;
     // the gathered form is built for the MoE expert layout: one token, split bf16 S and B
     if (gsel != nullptr && (batch != 1 || interleaved || meta_kind != 1)) return hipErrorInvalidValue;
-    for (uint32_t t0 = 0; t0 < batch;) {
-        uint32_t nb = batch - t0 >= kMaxNB ? kMaxNB : batch - t0;
-        VPlan pl;
-        while (!make_vplan(M, K, nb, cfg, pl)) {  // x of nb tokens too large for LDS
-            if (nb == 1) return hipErrorInvalidValue;
-            nb = nb > 2 ? 2 : 1;
-        }
+    if (ps.n == 0) return hipErrorInvalidValue;
+    for (uint32_t t0 = 0, i = 0, left = ps.p[0].times; t0 < batch;) {
+        const VPlan& pl = ps.p[i].pl;
+        const uint32_t nb = ps.p[i].nb;
         VArgs a;
         a.W = W;
         a.S = S;
@@ -585,6 +584,7 @@ hipError_t launch_int4_valu(const uint32_t* W, const uint16_t* S, const uint16_t
                                              : vgo_nb<1>(a, pl, interleaved, bf, s);
         if (e != hipSuccess) return e;
         t0 += nb;
+        if (--left == 0 && t0 < batch) left = ps.p[++i].times;
     }
     return hipSuccess;
 }

@@ -19,8 +19,7 @@ namespace {
 
 constexpr size_t kLdsMax = 160 * 1024;
 
-bool make_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t ntok, Int4Cfg cfg, mfma::Plan& out) {
-    (void)ntok;
+bool make_plan(uint32_t M, uint32_t K, uint32_t G, Int4Cfg cfg, mfma::Plan& out) {
     const uint32_t nspan = K / 128, ntiles = (M + mfma::kTile - 1) / mfma::kTile, cu = cu_count();
     // cfg.unroll: 0 = automatic, or 10 * T + T's ring depth (12, 24, 42);
     // cfg.rows: K parts P (0 = automatic)
@@ -69,40 +68,29 @@ bool make_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t ntok, Int4Cfg cfg, m
 
 }  // namespace
 
-uint32_t int4_mfma_tokens_per_pass(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg) {
-    mfma::Plan pl;
-    return int4_mfma_supported(M, K, G, batch, cfg) && make_plan(M, K, G, batch, cfg, pl) ? batch : 0;
-}
-
 // The pass is bound by each wave's serial steps (dequant, MFMA chains,
 // epilogue), not by HBM at these sizes: ~0.42 us per (step x tile) at 8 waves
 // a CU, plus ~3.3 us of launch and ramp, ~2% more per token above 4 (fitted:
 // 1024x4096 .. 8192x28672 at 3-16 tokens).
-double int4_mfma_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg) {
-    mfma::Plan pl;
-    if (!make_plan(M, K, G, batch, cfg, pl)) return 1e30;
+double int4_mfma_us(const mfma::Plan& pl, uint32_t batch) {
     const uint32_t cu = cu_count();
     const double work = (double)pl.nsteps * pl.T * (pl.waves / 8.0) * ((pl.nwg + cu - 1) / cu);
     return 3.3 + 0.42 * work * (1.0 + 0.02 * ((double)batch - 4.0));
 }
 
-Int4Cfg int4_mfma_default(uint32_t, uint32_t, uint32_t) { return Int4Cfg{0, 0}; }
-
 // Buffer loads address with 32-bit offsets: W, the scales and x must each
 // span less than 2 GiB.
-bool int4_mfma_supported(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg) {
+bool int4_mfma_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, mfma::Plan& pl) {
     if (batch < 1 || batch > 16 || M == 0) return false;
     if (!(G == 32 || G == 64 || G == 128) || K % 128) return false;
     if ((uint64_t)M * K / 2 >= (1ull << 31)) return false;
-    mfma::Plan pl;
-    return make_plan(M, K, G, batch, cfg, pl);
+    return make_plan(M, K, G, cfg, pl);
 }
 
 hipError_t launch_int4_mfma(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                             bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
-                            uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, hipStream_t s) {
-    mfma::Plan pl;
-    if (!make_plan(M, K, G, batch, cfg, pl)) return hipErrorInvalidValue;
+                            uint32_t K, uint32_t G, uint32_t batch, const mfma::Plan& pl,
+                            hipStream_t s) {
     mfma::Args a;
     a.W = W;
     a.S = S;

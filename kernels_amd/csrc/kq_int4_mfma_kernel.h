@@ -91,12 +91,6 @@ struct Args {
     uint32_t part_bytes;         // LDS of the K-part reduction (the weight staging follows)
 };
 
-// Launch plan chosen on the host.
-struct Plan {
-    uint32_t T, P, Q, J, J8, rounds, groups_wg, nwg, nsteps, waves;
-    size_t lds;
-};
-
 // Waves per workgroup that the register budget of (G, T, D) allows without
 // spills: 16 waves leave 128 registers per lane, 8 leave 256.
 __host__ __device__ constexpr uint32_t max_waves(uint32_t G, uint32_t T) {

@@ -17,15 +17,27 @@ struct Int4Cfg {
 // Compute units of the current device (queried once; 256 if the query fails).
 uint32_t cu_count();
 
-// Default launch shape for a problem (tuning table).
-Int4Cfg int4_valu_default(uint32_t M, uint32_t K, uint32_t batch);
+// Launch plan of one pass of the vector path (kq_int4.hip, make_vplan).
+struct VPlan {
+    uint32_t R, P, Q, J, rounds, groups_wg, nwg, nreal, nsteps, D, xw;
+    size_t lds;
+};
+// The passes of a call: `times` of `nb` tokens on one plan each, in order.
+struct Int4Passes {
+    struct {
+        uint32_t nb, times;
+        VPlan pl;
+    } p[4];
+    uint32_t n;  // 0: no plan
+};
+Int4Passes int4_valu_passes(uint32_t M, uint32_t K, uint32_t batch, Int4Cfg cfg);
 size_t int4_valu_lds_bytes(uint32_t K, uint32_t batch);
-// `batch` tokens on the vector path in batch-1-pass units x 100 (AUTO's crossover).
-uint32_t int4_valu_cost(uint32_t M, uint32_t K, uint32_t batch);
-// Modelled duration (us) of `batch` tokens on the vector path (AUTO's
-// crossovers, with int4_mfma and with the skinny kernels).
-double int4_valu_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch);
-double int4_valu_pass_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch);
+// The passes in batch-1-pass units x 100 (AUTO's crossover).
+uint32_t int4_valu_cost(const Int4Passes& ps);
+// Their modelled duration (us; AUTO's crossovers, with int4_mfma and with the
+// skinny kernels).
+double int4_valu_us(const Int4Passes& ps, uint32_t M, uint32_t K, uint32_t G);
+double int4_valu_pass_us(const Int4Passes& ps, uint32_t M, uint32_t K, uint32_t G);
 
 // gsel (device pointer, may be null): the kernel reads the matrix index
 // gsel[0] and moves W, S and B by gsel[0] * gstride bytes -- one matrix of a
@@ -33,19 +45,25 @@ double int4_valu_pass_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch);
 // take one token and split bf16 S and B (the MoE expert layout).
 hipError_t launch_int4_valu(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                             bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
-                            uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, hipStream_t s,
-                            const uint32_t* gsel = nullptr, uint64_t gstride = 0);
-bool int4_valu_supported(uint32_t K, uint32_t batch, Int4Cfg cfg);
+                            uint32_t K, uint32_t G, uint32_t batch, const Int4Passes& ps,
+                            hipStream_t s, const uint32_t* gsel = nullptr, uint64_t gstride = 0);
+bool int4_valu_supported(uint32_t K, Int4Cfg cfg);
 
+// Launch plan of the matrix-core path (kq_int4_mfma.hip); false: a shape or a
+// forced cfg it does not take.
+namespace mfma {
+struct Plan {
+    uint32_t T, P, Q, J, J8, rounds, groups_wg, nwg, nsteps, waves;
+    size_t lds;
+};
+}  // namespace mfma
+bool int4_mfma_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, mfma::Plan& pl);
 hipError_t launch_int4_mfma(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                             bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
-                            uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg, hipStream_t s);
-bool int4_mfma_supported(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg);
-Int4Cfg int4_mfma_default(uint32_t M, uint32_t K, uint32_t batch);
-// Tokens one matrix-core pass takes (all of them; 0: the shape is not supported).
-uint32_t int4_mfma_tokens_per_pass(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg);
-// Modelled duration (us) of one matrix-core pass (AUTO's crossover).
-double int4_mfma_us(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, Int4Cfg cfg);
+                            uint32_t K, uint32_t G, uint32_t batch, const mfma::Plan& pl,
+                            hipStream_t s);
+// Modelled duration (us) of a matrix-core pass, of all tokens (AUTO's crossover).
+double int4_mfma_us(const mfma::Plan& pl, uint32_t batch);
 
 // Skinny matrix-core kernels (kq_skinny.hip), 1-16 tokens in one pass: the
 // launch plan (false: a shape they don't take), its modelled duration, and

@@ -154,7 +154,8 @@ hipError_t launch_moe_unfused(const uint8_t* pool, const kq_moe_desc& d, const v
     float* V = reinterpret_cast<float*>(w + L.v);
     float* acc = reinterpret_cast<float*>(w + L.acc);
     const uint16_t* x = x_f32 ? xh : reinterpret_cast<const uint16_t*>(X);
-    const Int4Cfg auto_cfg{0, 0};
+    const Int4Passes pgu = int4_valu_passes(d.inter, d.hidden, 1, Int4Cfg{0, 0});
+    const Int4Passes pdn = int4_valu_passes(d.hidden, d.inter, 1, Int4Cfg{0, 0});
     hipError_t e;
 
     if ((e = launch_moe_logits(R, r_f32, X, x_f32, 1, d, xh, lg, s)) != hipSuccess) return e;
@@ -165,25 +166,26 @@ hipError_t launch_moe_unfused(const uint8_t* pool, const kq_moe_desc& d, const v
 
     // one projection of expert idx[slot]: W, S, B of expert 0, moved on the device
     auto proj = [&](uint64_t off, const uint16_t* xin, float* yout, uint32_t M, uint32_t K,
-                    uint32_t slot) {
+                    const Int4Passes& ps, uint32_t slot) {
         const uint8_t* p = pool + off;
         return launch_int4_valu(reinterpret_cast<const uint32_t*>(p + d.sub_w),
                                 reinterpret_cast<const uint16_t*>(p + d.sub_s),
                                 reinterpret_cast<const uint16_t*>(p + d.sub_b), 1, false, xin,
-                                yout, true, M, K, 64, 1, auto_cfg, s, idx + slot, d.blob);
+                                yout, true, M, K, 64, 1, ps, s, idx + slot, d.blob);
     };
     const uint32_t gi = (d.inter + kUThreads - 1) / kUThreads;
     const uint32_t gh = (d.hidden + kUThreads - 1) / kUThreads;
     for (uint32_t k = 0; k < d.top_k; ++k) {
-        if ((e = proj(d.off_gate, x, G, d.inter, d.hidden, k)) != hipSuccess) return e;
-        if ((e = proj(d.off_up, x, U, d.inter, d.hidden, k)) != hipSuccess) return e;
+        if ((e = proj(d.off_gate, x, G, d.inter, d.hidden, pgu, k)) != hipSuccess) return e;
+        if ((e = proj(d.off_up, x, U, d.inter, d.hidden, pgu, k)) != hipSuccess) return e;
         u_swiglu_k<<<gi, kUThreads, 0, s>>>(G, U, pool, d.blob, d.off_gate + d.sub_bi,
                                             d.off_up + d.sub_bi, idx + k,
                                             H + (size_t)k * d.inter, d.inter);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     for (uint32_t k = 0; k < d.top_k; ++k) {
-        if ((e = proj(d.off_down, H + (size_t)k * d.inter, V, d.hidden, d.inter, k)) != hipSuccess)
+        if ((e = proj(d.off_down, H + (size_t)k * d.inter, V, d.hidden, d.inter, pdn, k)) !=
+            hipSuccess)
             return e;
         u_axpy_k<<<gh, kUThreads, 0, s>>>(V, pool, d.blob, d.off_down + d.sub_bi, idx + k, wgt, k,
                                           acc, Y, y_f32 ? 1 : 0, k + 1 == d.top_k ? 1 : 0,
