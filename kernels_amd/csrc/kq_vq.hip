@@ -542,28 +542,32 @@ double passes_us(const QPass* ps, uint32_t n, uint32_t K) {
 // limit it: 3 tokens (two passes) 4096x4096 passes 9.3 / skinny 5.5 us, but
 // 300x28672 13.5 / 15.0; 4 tokens (one pass) 4096x4096 6.7 / 5.6, 700x608 4.9 /
 // 3.7, but 1940x3488 5.3 / 6.1; 2 tokens 28672x512 10.5 / 5.7, but 4096x4096 5.3 /
-// 5.5. Then the modelled durations decide: codebook blocks whose tiles divide
-// badly leave few workgroups there (11008x4096, a codebook per 1376 rows, 4
-// tokens: 12.4 us in passes, 67 on 16 workgroups; 28672x8192, per 4112, 8 tokens:
-// 99 / 719), while 9 tokens of 14336x4096 (per 256) take 36.4 / 13.8 and 5 of
-// 300x28672 (one codebook) 20.2 / 15.2.
+// 5.5. From 5 tokens tiles spread evenly over the CUs always win (809 calls; 9
+// tokens of 14336x4096, a codebook per 256 rows, 36.4 / 13.8, 5 of 300x28672 20.2 /
+// 15.2), and the passes are not planned. Else the modelled durations decide:
+// codebook blocks whose tiles divide badly leave few workgroups there
+// (11008x4096, per 1376 rows, 4 tokens: 12.4 us in passes, 67 on 16 workgroups;
+// 28672x8192, per 4112, 8 tokens: 99 / 719). n: the passes planned, 0 if not.
 namespace {
 bool skinny_pays(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch,
-                 const QPass* ps, uint32_t n, skinny::Plan& sp) {
+                 skinny::Plan& sp, QPass (&ps)[3], uint32_t& n) {
     const uint32_t cu = cu_count(), ntiles = (M + 15) / 16;
+    n = 0;
     if (batch < 2 || (batch == 2 && (ntiles <= cu || K > 2048)) ||
         (batch == 3 && ntiles * 8 < cu && K > 8192) || (batch == 4 && ntiles * 2 < cu && K > 2048))
         return false;
-    return vq_skinny_plan(M, K, rows_per_cb, scale_group, batch, sp) &&
-           0.95 * vq_skinny_us(sp, K, scale_group, batch) < passes_us(ps, n, K);
+    if (!vq_skinny_plan(M, K, rows_per_cb, scale_group, batch, sp)) return false;
+    if (batch >= 5 && sp.tiles_wg == (ntiles + cu - 1) / cu) return true;
+    n = make_qpasses(M, K, batch, rows_per_cb, ps);
+    return 0.95 * vq_skinny_us(sp, K, scale_group, batch) < passes_us(ps, n, K);
 }
 }  // namespace
 
 bool vq_takes_skinny(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scale_group, uint32_t batch) {
     QPass ps[3];
     skinny::Plan sp;
-    const uint32_t n = make_qpasses(M, K, batch, rows_per_cb, ps);
-    return n != 0 && skinny_pays(M, K, rows_per_cb, scale_group, batch, ps, n, sp);
+    uint32_t n;
+    return skinny_pays(M, K, rows_per_cb, scale_group, batch, sp, ps, n);
 }
 
 bool vq_supported(uint32_t M, uint32_t K, uint32_t rows_per_cb) {
@@ -575,11 +579,11 @@ hipError_t launch_vq(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, c
                      void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                      uint32_t scale_group, uint32_t batch, hipStream_t s) {
     QPass ps[3];
-    const uint32_t n = make_qpasses(M, K, batch, rows_per_cb, ps);
-    if (n == 0) return hipErrorInvalidValue;
+    uint32_t n;
     skinny::Plan sp;
-    if (skinny_pays(M, K, rows_per_cb, scale_group, batch, ps, n, sp) && vq_skinny_usable(K, scale_group))
+    if (skinny_pays(M, K, rows_per_cb, scale_group, batch, sp, ps, n) && vq_skinny_usable(K, scale_group))
         return launch_vq_skinny(IDX, C, S, X, Y, y_f32, M, K, rows_per_cb, scale_group, batch, sp, s);
+    if (n == 0 && (n = make_qpasses(M, K, batch, rows_per_cb, ps)) == 0) return hipErrorInvalidValue;
     uint32_t sgs = 0;
     while ((1u << sgs) < scale_group) ++sgs;
     const bool per_row = scale_group == K;
