@@ -174,6 +174,8 @@ kq_status kq_vq_gemv(const uint8_t* IDX, const uint16_t* C, const uint16_t* S,
  * their group's scale -- all of the block's pairs, or `sample` of them drawn
  * with replacement when there are more -- 256 initial centroids drawn from
  * that sample, `iters` iterations, then every pair to its nearest centroid.
+ * A codeword is fp16 of the mean of its points, rounded once (from the double,
+ * not through the fp32 centroid that the searches use).
  * The draws are seeded (splitmix64 of seed, block and draw number) and the
  * cluster sums are exact integer sums, so the output is a function of the
  * arguments (the same on every run and device).

@@ -21,7 +21,8 @@
 //    depend on their order) and each centroid moves to its mean (empty
 //    clusters stay).
 // 4. every pair of every row goes to its block's nearest fp32 centroid
-//    (pq_quantize.py:66-73); the codebook is stored as fp16.
+//    (pq_quantize.py:66-73); the codebook is stored as fp16, rounded from the
+//    means (a centroid that never moved: from its sample point).
 //
 // The nearest-centroid searches are all of the work: 256 scores for each of
 // 25 x 200,000 sample points a block and then for every pair. Points lie in
@@ -226,17 +227,24 @@ __global__ __launch_bounds__(kQT) void vq_km_assign_k(const float2* __restrict__
     }
 }
 
+// A moved centroid: fp32 for the next searches, and its codeword, rounded to fp16
+// once from the mean itself (through the fp32 centroid, ties of that rounding's
+// making would round twice).
+__device__ __forceinline__ void vq_store_mean(double x, double y, size_t i, float2* cent,
+                                              uint16_t* Cb) {
+    cent[i] = make_float2((float)x, (float)y);
+    Cb[2 * i] = __builtin_bit_cast(uint16_t, (_Float16)x);
+    Cb[2 * i + 1] = __builtin_bit_cast(uint16_t, (_Float16)y);
+}
+
 __global__ __launch_bounds__(kQT) void vq_km_update_k(VqAcc* __restrict__ acc,
                                                       float2* __restrict__ cent,
                                                       uint16_t* __restrict__ Cb) {
     const size_t i = (size_t)blockIdx.x * kCB + threadIdx.x;
     const VqAcc q = acc[i];
     if (q.n != 0) {
-        const float2 v = make_float2((float)((double)(long long)q.x * 0x1p-40 / (double)q.n),
-                                     (float)((double)(long long)q.y * 0x1p-40 / (double)q.n));
-        cent[i] = v;
-        Cb[2 * i] = f2h(v.x);
-        Cb[2 * i + 1] = f2h(v.y);
+        vq_store_mean((double)(long long)q.x * 0x1p-40 / (double)q.n,
+                      (double)(long long)q.y * 0x1p-40 / (double)q.n, i, cent, Cb);
     }
     acc[i] = VqAcc{0, 0, 0};
 }
@@ -358,14 +366,8 @@ __global__ __launch_bounds__(kCellT) void vq_cells_k(const uint8_t* __restrict__
                 const double ax = (double)(long long)x * 0x1p-40 / (double)n;
                 const double ay = (double)(long long)y * 0x1p-40 / (double)n;
                 v = make_float2((float)ax, (float)ay);
-                if (blockIdx.x == 0) {  // the others use cent[ci] only where n is 0
-                    cent[ci] = v;
-                    // one rounding from the mean, as the full scan's update
-                    // compiles to: through the float, ties of its own making
-                    // would round twice
-                    Cb[2 * ci] = __builtin_bit_cast(uint16_t, (_Float16)ax);
-                    Cb[2 * ci + 1] = __builtin_bit_cast(uint16_t, (_Float16)ay);
-                }
+                // the other workgroups use cent[ci] only where n is 0
+                if (blockIdx.x == 0) vq_store_mean(ax, ay, ci, cent, Cb);
             }
         }
         cs[t] = v;

@@ -68,6 +68,8 @@ def lib():
         L.kqref_vq_fix.restype = C.c_int64
         L.kqref_vq_mean.argtypes = [C.c_int64, C.c_uint64]
         L.kqref_vq_mean.restype = C.c_float
+        L.kqref_vq_codeword.argtypes = [C.c_int64, C.c_uint64]
+        L.kqref_vq_codeword.restype = C.c_uint16
         _lib = L
     return _lib
 

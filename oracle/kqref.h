@@ -123,6 +123,7 @@ uint64_t kqref_vq_hash(uint64_t seed, uint32_t blk, uint32_t j);
 float kqref_vq_score(float px, float py, float cx, float cy);
 int64_t kqref_vq_fix(float v);
 float kqref_vq_mean(int64_t sum, uint64_t cnt);
+uint16_t kqref_vq_codeword(int64_t sum, uint64_t cnt);
 
 #ifdef __cplusplus
 }

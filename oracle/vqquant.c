@@ -23,7 +23,9 @@
  *      GPU's atomics -- cannot change the result): mean =
  *      (float)((double)sum * 2^-40 / count), coordinates truncated to the grid.
  *   4. every pair of the block is assigned with the fp32 centroids
- *      (pq_quantize.py:66-73); the codebook is stored as fp16 (RNE).
+ *      (pq_quantize.py:66-73); the codebook is stored as fp16 (RNE), rounded
+ *      once from the double mean (not through the fp32 centroid), from the
+ *      sample point where a cluster never had points.
  */
 #include <math.h>
 #include <stdint.h>
@@ -72,9 +74,26 @@ static uint32_t nearest(float px, float py, const float* C) {
 
 int64_t kqref_vq_fix(float v) { return (int64_t)(v * 0x1p40f); }
 
-float kqref_vq_mean(int64_t sum, uint64_t cnt) {
-    return (float)((double)sum * 0x1p-40 / (double)cnt);
+static double mean64(int64_t sum, uint64_t cnt) { return (double)sum * 0x1p-40 / (double)cnt; }
+
+float kqref_vq_mean(int64_t sum, uint64_t cnt) { return (float)mean64(sum, cnt); }
+
+/* fp16 of a double, rounded once: the double is first cut to a float whose last
+ * bit says whether anything was cut off (rounding to odd), which leaves fp16's
+ * rounding the same decision. */
+static uint16_t f64_to_f16(double d) {
+    float f = (float)d;
+    if ((double)f != d) {
+        uint32_t b;
+        memcpy(&b, &f, 4);
+        if (fabs((double)f) > fabs(d)) --b;
+        b |= 1;
+        memcpy(&f, &b, 4);
+    }
+    return kqref_f32_to_f16(f);
 }
+
+uint16_t kqref_vq_codeword(int64_t sum, uint64_t cnt) { return f64_to_f16(mean64(sum, cnt)); }
 
 void kqref_vq_quantize(const void* W, int w_dtype, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                        uint32_t scale_group, uint32_t iters, uint32_t sample, uint64_t seed,
@@ -114,6 +133,8 @@ void kqref_vq_quantize(const void* W, int w_dtype, uint32_t M, uint32_t K, uint3
             C[2 * c] = P[2 * j];
             C[2 * c + 1] = P[2 * j + 1];
         }
+        uint16_t* H = Cb + (size_t)b * 2 * KQREF_CB;
+        for (uint32_t c = 0; c < 2 * KQREF_CB; ++c) H[c] = kqref_f32_to_f16(C[c]);
         int64_t sx[KQREF_CB], sy[KQREF_CB];
         uint64_t cnt[KQREF_CB];
         for (uint32_t it = 0; it < iters; ++it) {
@@ -130,13 +151,13 @@ void kqref_vq_quantize(const void* W, int w_dtype, uint32_t M, uint32_t K, uint3
                 if (cnt[c]) {
                     C[2 * c] = kqref_vq_mean(sx[c], cnt[c]);
                     C[2 * c + 1] = kqref_vq_mean(sy[c], cnt[c]);
+                    H[2 * c] = kqref_vq_codeword(sx[c], cnt[c]);
+                    H[2 * c + 1] = kqref_vq_codeword(sy[c], cnt[c]);
                 }
         }
         free(P);
-        for (uint32_t c = 0; c < 2 * KQREF_CB; ++c) {
-            Cb[(size_t)b * 2 * KQREF_CB + c] = kqref_f32_to_f16(C[c]);
-            if (centroids_out) centroids_out[(size_t)b * 2 * KQREF_CB + c] = C[c];
-        }
+        if (centroids_out)
+            memcpy(centroids_out + (size_t)b * 2 * KQREF_CB, C, sizeof C);
         for (uint32_t m = r0; m < r0 + rows; ++m)
             for (uint32_t i = 0; i < half; ++i) {
                 float px, py;

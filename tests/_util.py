@@ -54,3 +54,16 @@ def inf_rel(got, ref):
     got = np.asarray(got, np.float64)
     ref = np.asarray(ref, np.float64)
     return float(np.max(np.abs(got - ref)) / max(1e-30, np.max(np.abs(ref))))
+
+
+def tie_weights(M, K, seed):
+    """Weights [M][K] float32 (for one scale per row: every row's is 1) whose
+    pairs crowd 144 places with coordinates halfway between two fp16 values, or
+    one float32 step above: cluster means lie a fraction of a step above the
+    tie, where rounding through float32 goes the other way."""
+    rng = np.random.default_rng(seed)
+    tie = (0.5 + (4 * np.arange(12) * 40 + 1) * 2.0**-12).astype(np.float32)
+    W = rng.choice(tie, (M, K)).astype(np.float32)
+    W += (rng.random((M, K)) < 0.3).astype(np.float32) * np.float32(2.0**-24)
+    W[:, :2] = 1.0
+    return W

@@ -10,7 +10,7 @@ import torch
 
 import oracle
 from kernels_amd import kq
-from tests._util import assert_close, dev, host_bits, to_f64
+from tests._util import assert_close, dev, host_bits, tie_weights, to_f64
 
 pytestmark = pytest.mark.gpu
 
@@ -112,6 +112,19 @@ def test_quantize_zero_and_constant_rows(gpu):
     Wd = torch.from_numpy(W).to(gpu)
     IDX, Cb, S = quantize_gpu(gpu, Wd, M, K, 32, 32, 4, 900, 5)
     oIDX, oCb, oS, _ = oracle.vq_quantize(W, oracle.F32, M, K, 32, 32, iters=4, sample=900, seed=5)
+    assert np.array_equal(host_bits(S, np.uint16), oS)
+    assert np.array_equal(host_bits(Cb, np.uint16), oCb)
+    assert np.array_equal(IDX.cpu().numpy(), oIDX)
+
+
+# Codewords are rounded once from the double mean, in the full scan and with
+# cell lists of both sizes alike (clusters whose float32 mean is an fp16 tie).
+@pytest.mark.parametrize("M,K", [(32, 512), (64, 1024), (64, 4096)])
+def test_quantize_codewords_round_the_mean_once(gpu, M, K):
+    W = tie_weights(M, K, M + K)
+    IDX, Cb, S = quantize_gpu(gpu, torch.from_numpy(W).to(gpu), M, K, M, K, 3, 1 << 20, 0)
+    oIDX, oCb, oS, cent = oracle.vq_quantize(W, oracle.F32, M, K, M, K, iters=3, sample=1 << 20)
+    assert np.sum(oCb != cent.astype(np.float16).view(np.uint16)) > 20
     assert np.array_equal(host_bits(S, np.uint16), oS)
     assert np.array_equal(host_bits(Cb, np.uint16), oCb)
     assert np.array_equal(IDX.cpu().numpy(), oIDX)

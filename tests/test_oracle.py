@@ -16,6 +16,7 @@ import pytest
 
 import oracle
 from kernels_amd import gen
+from tests._util import tie_weights
 
 GOLD = os.path.join(os.path.dirname(__file__), "golden")
 
@@ -429,6 +430,25 @@ def test_vq_quant_lloyd_matches_numpy():
             _, _, _, got = oracle.vq_quantize(W, oracle.F32, M, K, M, 32, iters=it,
                                               sample=1 << 20)
             assert np.max(np.abs(got[0] - C)) < 1e-6, it
+
+
+def test_vq_quant_codewords_round_the_mean_once():
+    """Codewords are fp16 of the double mean, not of the float32 centroid:
+    against numpy's own sums and float64 -> float16 rounding, on clusters whose
+    float32 mean is an fp16 tie and the double mean is not."""
+    M, K, n = 32, 512, 3
+    W = tie_weights(M, K, 5)
+    run = lambda it: oracle.vq_quantize(W, oracle.F32, M, K, M, K, iters=it, sample=1 << 20)  # noqa: E731
+    _, Cb, _, cent = run(n)
+    a = run(n - 1)[0].reshape(-1)  # every pair is sampled: the last iteration's assignment
+    fix = (W.reshape(-1, 2).astype(np.float64) * 2.0**40).astype(np.int64)
+    once = Cb[0].copy()
+    for c in np.unique(a):
+        sel = fix[a == c]
+        once[c] = (sel.sum(0).astype(np.float64) * 2.0**-40 / len(sel)).astype(np.float16).view(np.uint16)
+    twice = cent[0].astype(np.float16).view(np.uint16)
+    assert np.array_equal(Cb[0], once)
+    assert np.sum(once != twice) > 20  # the case tells the two apart
 
 
 def test_vq_quant_reconstruction_quality():
