@@ -124,6 +124,8 @@ hipError_t launch_moe_router(const void* R, bool r_f32, const void* X, bool x_f3
                              void* ws, hipStream_t s);
 hipError_t launch_moe_gate_up(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                               const uint16_t* xh, uint16_t* H, uint32_t batch, hipStream_t s);
+// Whether it runs the expert-partitioned kernel.
+bool moe_gate_up_partitions(const kq_moe_desc& d, uint32_t batch);
 hipError_t launch_moe_down(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                            const float* wgt, const uint16_t* H, void* Y, bool y_f32,
                            uint32_t batch, void* ws, hipStream_t s);  // ws: workspace or null

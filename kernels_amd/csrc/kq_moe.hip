@@ -32,12 +32,12 @@
 //      expert with only that expert's activations in LDS; down writes
 //      per-slot products to the workspace and a small moe_combine_k launch
 //      sums them in slot order (4 launches in all);
-//      The standalone entry points run them too, on the caller's idx (down
-//      where it has a workspace).
-//    - per tile (moe_gate_up_k, moe_down_k): shapes past the LDS limits and
-//      a standalone down without a workspace: a grid of (16-row tile,
-//      expert) or 8-output-row workgroups that issue all of their loads in
-//      one round trip.
+//      The standalone entry points run them too, on the caller's idx (gate/up
+//      where moe_gate_up_partitions says so, down where it has a workspace).
+//    - per tile (moe_gate_up_k, moe_down_k): shapes past the LDS limits, the
+//      other standalone gate/up calls from 3 tokens and a standalone down
+//      without a workspace: a grid of (16-row tile, expert) or 8-output-row
+//      workgroups that issue all of their loads in one round trip.
 //    Every form reads each selected expert's rows once per call for all
 //    token slots that chose it; a half-wave owns one row of a pair (gate /
 //    up, or two down rows; K = 2880 = 90 chunks -> 3 per lane), so SwiGLU
@@ -2615,14 +2615,37 @@ bool gu_part_ok(const kq_moe_desc& d, uint32_t batch) {
            d.blob < (1ull << 31) && st_act_bytes(batch, d.hidden) + kStStatic <= kLdsMax;
 }
 
+}  // namespace
+
+// Which standalone gate/up calls (the caller's idx) the partitioned kernel
+// takes. Every workgroup builds the plan there and stages every token's x
+// before its first row, 2-3 us that the block's form hides behind its router:
+// it pays where the rows of the distinct experts (their number with even
+// routing), or the slots' h values, are many. Against streaming at 2 tokens
+// (fitted on 1511 calls): 1024x1024, 1 of 8 experts 3.7 streaming / 5.4 us
+// partitioned, 2880x2880, 4 of 128 19.8 / 19.1. Against the per-tile kernel
+// (3487 calls), a few slots a row cost its waves little while x is at most 1024
+// long: 704x2304, 1 of 82, 12 tokens 9.6 per tile / 15.0, but 2880x2880, 4 of
+// 128, 16 tokens 144 / 89. The last constants keep near ties where they are: 0.5%
+// of the calls lose more than 6% by the rule, the mean gains 12%.
+bool moe_gate_up_partitions(const kq_moe_desc& d, uint32_t batch) {
+    if (batch < 2 || !gu_part_ok(d, batch)) return false;
+    double rest = 1.0;  // share of the experts that no token chose
+    for (uint32_t t = 0; t < batch; ++t) rest *= 1.0 - (double)d.top_k / d.n_experts;
+    const double J = chunks_j(d.hidden), rows = d.n_experts * (1.0 - rest) * d.inter / 1e3;
+    const double hs = (double)batch * d.top_k * d.inter / 1e3;
+    if (gu_streams(d, batch)) return 0.133 * rows > 2.0 + 0.31 * J;
+    return J * (0.07 * rows + 0.095 * hs - 0.46) > 0.23 * rows + 0.058 * hs + 1.0;
+}
+
+namespace {
+
 template <bool FP>
 hipError_t launch_gu(const uint8_t* pool, const kq_moe_desc& d, const uint32_t* idx,
                      const Plan* plan, const uint16_t* xh, uint16_t* H, uint32_t batch,
                      hipStream_t s) {
     if constexpr (!FP) {
-        // the block's choice (block_gu_streams); 16 tokens at gpt-oss-120b
-        // shapes: per tile 147 us, partitioned 87 us
-        if (!block_gu_streams(d, batch) && gu_part_ok(d, batch))
+        if (moe_gate_up_partitions(d, batch))
             return launch_gu_part<true>(pool, d, xh, H, batch,
                                         GuTopk{nullptr, const_cast<uint32_t*>(idx), nullptr, nullptr}, s);
     }

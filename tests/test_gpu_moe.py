@@ -227,6 +227,24 @@ def test_standalone_repeated_experts(gpu, slot_pools, tk, batch, kind):
         assert_close(to_f64(b.y), Yref, atol=1e-4, rtol=1e-4, what=f"down {wsb}")
 
 
+# A caller's routing with every expert shared and named twice a token, at
+# shapes that the partitioned gate/up takes (test_routes.py): the plan from idx
+# with entries cut to a token's slots, x of one to four chunks a lane.
+@pytest.mark.parametrize("hidden,inter,ne,tk,batch", [(3072, 512, 8, 8, 16), (4096, 512, 8, 8, 12),
+                                                      (1024, 1024, 8, 8, 16), (1536, 2048, 12, 4, 9)])
+def test_standalone_gate_up_partitioned_repeats(gpu, hidden, inter, ne, tk, batch):
+    d, off = _compact_desc(hidden, inter, ne, tk)
+    host = gen.moe_pool(ne, seed=hidden, quantize=True, hidden=hidden, inter=inter, blob=d.blob, off=off)
+    rng = np.random.default_rng(batch)
+    idx = rng.integers(0, ne, (batch, tk)).astype(np.uint32)
+    idx[0] = 3
+    X = gen.f16_bits(rng.normal(0, 1, (batch, hidden)))
+    b = Block(gpu, d, batch)
+    kq.moe_gate_up_swiglu(dev(host, gpu), d, dev(idx, gpu), dev(X, gpu), b.H, b.ws, b.wsb, batch=batch)
+    torch.cuda.synchronize()
+    assert_close(to_f64(b.H), oracle.moe_gate_up(host, odesc(d), idx, X, oracle.F16, batch), what="h")
+
+
 def test_duplicate_and_shared_experts(gpu, pool16):
     """Slots that select the same expert (within and across tokens) read its
     rows once and still land in their own h / y slots."""
