@@ -45,47 +45,43 @@ kq_status check_int4(const uint32_t* W, const void* S, const void* B, kq_dtype s
     return KQ_OK;
 }
 
-kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_dtype,
-                   const uint16_t* X, void* Y, kq_dtype y_dtype, uint32_t M, uint32_t K,
-                   uint32_t G, uint32_t batch, kq_int4_path path, const kq::Int4Cfg* forced,
-                   kq_stream_t stream) {
-    kq_status st = check_int4(W, S, B, sb_dtype, X, Y, y_dtype, M, K, G, batch);
-    if (st != KQ_OK) return st;
-    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const int mk = sb_dtype == KQ_BF16 ? 1 : 0;
-    const bool inter = B == nullptr;
-    const auto* Sp = static_cast<const uint16_t*>(S);
-    const auto* Bp = static_cast<const uint16_t*>(B);
-    const bool yf = y_dtype == KQ_F32;
-
-    // the plan of each path that the call may take, made once
-    const kq::Int4Cfg cfg = forced ? *forced : kq::Int4Cfg{0, 0};
+// The plans of an int4 call's paths, each made once.
+struct Int4Plans {
     kq::Int4Passes vp;
-    vp.n = 0;
+    kq::mfma::Plan mp;
+    kq::skinny::Plan sp;
+};
+
+// The path an int4 call takes (kq::kPathSkinny: the skinny matrix-core kernels),
+// and its plan; KQ_PATH_AUTO: none of the paths asked for takes it. meta8:
+// scales and biases start at multiples of 8 bytes.
+int choose_int4(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, bool meta8, int path,
+                const kq::Int4Cfg* forced, Int4Plans& p) {
+    if (path == KQ_PATH_SCALAR) return path;
+    const kq::Int4Cfg cfg = forced ? *forced : kq::Int4Cfg{0, 0};
     bool valu_ok = false;
     if (path == KQ_PATH_AUTO || path == KQ_PATH_VALU) {
-        vp = kq::int4_valu_passes(M, K, batch, cfg);
-        valu_ok = forced ? kq::int4_valu_supported(K, cfg) : vp.n != 0;
+        p.vp = kq::int4_valu_passes(M, K, batch, cfg);
+        valu_ok = forced ? kq::int4_valu_supported(K, cfg) : p.vp.n != 0;
     }
     // one token is the vector path's (its cost is the crossover's unit, 100
     // against 120); the other paths' plans are not looked at (1.5 us of host
     // time a call)
     if (path == KQ_PATH_AUTO && batch == 1 && valu_ok) path = KQ_PATH_VALU;
+    if (path == KQ_PATH_VALU) return valu_ok ? path : KQ_PATH_AUTO;
     // the matrix-core path reads a span's separate scales / biases as one
     // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
     // last two spans: with an odd number of spans that word would end past the
     // array, and the range check would zero it
-    kq::mfma::Plan mp;
-    const bool mfma_shape = (path == KQ_PATH_AUTO || path == KQ_PATH_MFMA) &&
-                            (inter || (aligned(S, 8) && aligned(B, 8))) &&
-                            kq::int4_mfma_plan(M, K, G, batch, cfg, mp);
+    const bool mfma_shape = (inter || meta8) && kq::int4_mfma_plan(M, K, G, batch, cfg, p.mp);
     const bool mfma_ok = mfma_shape && (inter || G != 128 || (K / 128) % 2 == 0);
     // ... those go to the skinny kernels where the matrix cores are asked for, or
     // the only path that takes K
-    kq::skinny::Plan sp;
-    if (mfma_shape && !mfma_ok && (path == KQ_PATH_MFMA || (path == KQ_PATH_AUTO && !valu_ok)) &&
-        kq::int4_skinny_plan(M, K, G, batch, inter, sp))
-        return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
+    if (mfma_shape && !mfma_ok && (path == KQ_PATH_MFMA || !valu_ok) &&
+        kq::int4_skinny_plan(M, K, G, batch, inter, p.sp))
+        return kq::kPathSkinny;
+    if (path == KQ_PATH_MFMA) return mfma_ok ? path : KQ_PATH_AUTO;
+    if (!valu_ok && !mfma_ok) return KQ_PATH_AUTO;
     // Crossover, in batch-1 vector passes: a vector pass takes up to 4 tokens
     // (int4_valu_cost), a matrix-core pass all of them at ~1.2 (29.3-30.3 us
     // against 24.9 us at 28672 x 8192; 64-byte row pieces per load instead of
@@ -94,38 +90,51 @@ kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_
     // at least ~9 us (each wave's serial steps), so small matrices stay on the
     // vector path longer: both durations are modelled too (1024x4096: vector
     // up to 8 tokens, 4.1-9.1 against 9.2-9.9 us; 4096x4096 up to 4).
-    if (path == KQ_PATH_AUTO) {
-        if (!mfma_ok) {
-            path = KQ_PATH_VALU;
-        } else if (!valu_ok) {
-            path = KQ_PATH_MFMA;
-        } else {
-            const bool fewer_passes = 120 < kq::int4_valu_cost(vp);
-            const bool faster = kq::int4_mfma_us(mp, batch) < kq::int4_valu_us(vp, M, K, G);
-            path = fewer_passes && faster ? KQ_PATH_MFMA : KQ_PATH_VALU;
-        }
-        // the skinny matrix-core kernels, any K of at least 256 (shapes that
-        // neither path takes stay refused): against the
-        // matrix cores' choice by size (int4_skinny_beats_mfma), against the
-        // vector path by duration (4096x4096: vector 5.4, skinny 6.0 us at 3
-        // tokens, 6.4 and 6.0 at 4, 10.0 and 6.1 at 5)
-        if (batch > 1 && (valu_ok || mfma_ok) && kq::int4_skinny_plan(M, K, G, batch, inter, sp) &&
-            (path == KQ_PATH_MFMA
-                 ? kq::int4_skinny_beats_mfma(sp, M, G, batch, inter)
-                 : !valu_ok || kq::int4_skinny_us(sp, batch) < kq::int4_valu_pass_us(vp, M, K, G)))
-            return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, sp, s));
+    path = !mfma_ok ? KQ_PATH_VALU : KQ_PATH_MFMA;
+    if (valu_ok && mfma_ok) {
+        const bool fewer_passes = 120 < kq::int4_valu_cost(p.vp);
+        const bool faster = kq::int4_mfma_us(p.mp, batch) < kq::int4_valu_us(p.vp, M, K, G);
+        path = fewer_passes && faster ? KQ_PATH_MFMA : KQ_PATH_VALU;
     }
-    if (path == KQ_PATH_VALU) {
-        if (!valu_ok) return KQ_EUNSUPPORTED;
-        return hip_status(kq::launch_int4_valu(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, vp, s));
+    // the skinny matrix-core kernels, any K of at least 256 (shapes that neither
+    // path takes stay refused), where their modelled duration is below that of
+    // the path chosen so far (4096x4096, G 64: vector 5.4, skinny 6.0 us at 3
+    // tokens, 6.4 and 6.0 at 4; int4_mfma 10.3, skinny 5.9 at 8; 28672x8192 30.4
+    // and 37.8). Of 14300 measured calls 32 lose more than 6% by it and the mean
+    // has 1.69 times the speed; int4_mfma keeps ties, its model is the rougher one.
+    if (batch > 1 && kq::int4_skinny_plan(M, K, G, batch, inter, p.sp) &&
+        kq::int4_skinny_us(p.sp, G, batch, inter) <
+            (path == KQ_PATH_MFMA ? 0.95 * kq::int4_mfma_pass_us(p.mp, G, batch)
+                                  : kq::int4_valu_pass_us(p.vp, M, K, G)))
+        return kq::kPathSkinny;
+    return path;
+}
+
+kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_dtype,
+                   const uint16_t* X, void* Y, kq_dtype y_dtype, uint32_t M, uint32_t K,
+                   uint32_t G, uint32_t batch, kq_int4_path path, const kq::Int4Cfg* forced,
+                   kq_stream_t stream) {
+    kq_status st = check_int4(W, S, B, sb_dtype, X, Y, y_dtype, M, K, G, batch);
+    if (st != KQ_OK) return st;
+    if (path < KQ_PATH_AUTO || path > KQ_PATH_SCALAR) return KQ_EINVAL;
+    const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const int mk = sb_dtype == KQ_BF16 ? 1 : 0;
+    const bool inter = B == nullptr;
+    const auto* Sp = static_cast<const uint16_t*>(S);
+    const auto* Bp = static_cast<const uint16_t*>(B);
+    const bool yf = y_dtype == KQ_F32;
+    Int4Plans p;
+    switch (choose_int4(M, K, G, batch, inter, aligned(S, 8) && aligned(B, 8), path, forced, p)) {
+        case KQ_PATH_VALU:
+            return hip_status(kq::launch_int4_valu(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, p.vp, s));
+        case KQ_PATH_MFMA:
+            return hip_status(kq::launch_int4_mfma(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, p.mp, s));
+        case kq::kPathSkinny:
+            return hip_status(kq::launch_int4_skinny(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, p.sp, s));
+        case KQ_PATH_SCALAR:
+            return hip_status(kq::launch_int4_scalar(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, s));
+        default: return KQ_EUNSUPPORTED;
     }
-    if (path == KQ_PATH_MFMA) {
-        if (!mfma_ok) return KQ_EUNSUPPORTED;
-        return hip_status(kq::launch_int4_mfma(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, mp, s));
-    }
-    if (path == KQ_PATH_SCALAR)
-        return hip_status(kq::launch_int4_scalar(W, Sp, Bp, mk, inter, X, Y, yf, M, K, G, batch, s));
-    return KQ_EINVAL;
 }
 
 kq_status check_desc(const kq_moe_desc* d, uint32_t batch) {
@@ -178,6 +187,16 @@ uint32_t cu_count() {
                                                                                                    : 256;
     if (slot) slot->store(n, std::memory_order_relaxed);
     return (uint32_t)n;
+}
+}  // namespace kq
+
+namespace kq {
+int int4_route(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, bool meta8, int path,
+               skinny::Plan* sp) {
+    Int4Plans p;
+    const int r = choose_int4(M, K, G, batch, inter, meta8, path, nullptr, p);
+    if (sp && r == kPathSkinny) *sp = p.sp;
+    return r;
 }
 }  // namespace kq
 

@@ -62,12 +62,13 @@ hipError_t launch_int4_mfma(const uint32_t* W, const uint16_t* S, const uint16_t
                             bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
                             uint32_t K, uint32_t G, uint32_t batch, const mfma::Plan& pl,
                             hipStream_t s);
-// Modelled duration (us) of a matrix-core pass, of all tokens (AUTO's crossover).
+// Modelled duration (us) of a matrix-core pass, of all tokens (AUTO's
+// crossovers, with the vector path and with the skinny kernels).
 double int4_mfma_us(const mfma::Plan& pl, uint32_t batch);
+double int4_mfma_pass_us(const mfma::Plan& pl, uint32_t G, uint32_t batch);
 
 // Skinny matrix-core kernels (kq_skinny.hip), 1-16 tokens in one pass: the
-// launch plan (false: a shape they don't take), its modelled duration, and
-// whether it beats int4_mfma.
+// launch plan (false: a shape they don't take) and its modelled duration.
 namespace skinny {
 struct Plan {
     uint32_t T, P, Q, J, NP, rounds, tiles_wg, nwg;
@@ -75,8 +76,7 @@ struct Plan {
 };
 }  // namespace skinny
 bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl);
-double int4_skinny_us(const skinny::Plan& pl, uint32_t batch);
-bool int4_skinny_beats_mfma(const skinny::Plan& pl, uint32_t M, uint32_t G, uint32_t batch, bool inter);
+double int4_skinny_us(const skinny::Plan& pl, uint32_t G, uint32_t batch, bool inter);
 hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,
                               bool interleaved, const uint16_t* X, void* Y, bool y_f32, uint32_t M,
                               uint32_t K, uint32_t G, uint32_t batch, const skinny::Plan& pl,
@@ -90,6 +90,13 @@ bool vq_takes_skinny(uint32_t M, uint32_t K, uint32_t rows_per_cb, uint32_t scal
 hipError_t launch_vq_skinny(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, const uint16_t* X,
                             void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                             uint32_t scale_group, uint32_t batch, const skinny::Plan& pl, hipStream_t s);
+
+// The path an int4 call takes without a forced launch shape: KQ_PATH_*, or
+// kPathSkinny (its plan to sp, if given), KQ_PATH_AUTO where it is refused. meta8:
+// scales and biases start at multiples of 8 bytes.
+constexpr int kPathSkinny = 4;
+int int4_route(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, bool meta8, int path,
+               skinny::Plan* sp);
 
 // Debug scalar path: one thread per (row, token), plain chunk loop (v0).
 hipError_t launch_int4_scalar(const uint32_t* W, const uint16_t* S, const uint16_t* B,

@@ -119,30 +119,21 @@ static double skinny_us(const skinny::Plan& pl, uint32_t batch, double form) {
     return 3.2 + (double)pl.rounds * pl.J * (kStep[b][t] + kWaves[b][t] * fill) * form;
 }
 
-// (the choice against the vector path still goes by plan_us)
-double int4_skinny_us(const skinny::Plan& pl, uint32_t batch) { return plan_us(pl, batch); }
+// A step's cost by int4 layout (medians of 14000 calls, nine in ten within 15%): 8
+// groups a pair take more work for scales, four tiles of 64-wide groups' separate
+// scales spill.
+double int4_skinny_us(const skinny::Plan& pl, uint32_t G, uint32_t batch, bool inter) {
+    const bool two8 = inter && pl.T == 2 && batch <= 8;
+    double form = two8 ? 0.98 : 0.92;
+    if (G == 64) form = pl.T < 4 ? (two8 ? 1.07 : 1.03) : inter ? 1.1 : 1.6;
+    if (G == 32) form = !inter ? 1.08 : two8 ? 1.45 : 1.22;
+    return skinny_us(pl, batch, form) + (pl.T > 1 ? 0.3 : 0.0);
+}
 
 bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl) {
     if (batch < 1 || batch > 16 || !(G == 32 || G == 64 || G == 128) || K % G) return false;
     if (!inter && G == 32 && batch <= 8) return false;  // its windows spill
     return make_plan(M, K, batch, int4_tmax(G), even_share(M), 0, pl);
-}
-
-// Against the int4_mfma kernels, which have a ~9 us floor and stream large
-// matrices better: up to 60 (above 8 tokens 64) pairs of spans of 16-row tiles a
-// CU, 32 with 8 groups a pair. Measured, skinny / int4_mfma at 8 tokens:
-// 4096x4096 (16 pairs) 5.9 / 10.3 us, 6144x4096 (32) 7.4 / 10.9, 4096x14336
-// (56) 13.9 / 17.0, 14336x4096 (64) 13.0 / 12.5 (16 tokens: 13.6 / 14.9);
-// 5120x20480 (160) 30.6 / 26.7, 28672x8192 (224) 37.8 / 30.4. A quarter or more of the last round's
-// tiles empty costs that lead up to 8 tokens (11008x4096: 12.2 / 11.5). Above 8
-// tokens separate arrays of 128-wide groups win at up to two tiles a CU
-// whatever K (8192x28672: 39.5 / 47.0).
-bool int4_skinny_beats_mfma(const skinny::Plan& pl, uint32_t M, uint32_t G, uint32_t batch, bool inter) {
-    const uint32_t per = even_share(M);
-    if (!inter && G == 128 && batch > 8 && per <= 2) return true;
-    const uint32_t work = per * pl.NP;
-    if (work > (G == 32 ? 32u : batch > 8 ? 64u : 60u)) return false;
-    return batch > 8 || work <= 32 || per * 5 >= pl.rounds * pl.T * pl.Q * 4;
 }
 
 hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,

@@ -28,6 +28,37 @@ def test_vq_route_follows_the_plans_duration(M, K, rpc, skinny):
             assert vq_takes_skinny(M, K, rpc, sg, batch) == skinny, (sg, batch)
 
 
+VALU, MFMA, SKINNY = kq.PATH_VALU, kq.PATH_MFMA, 4
+REFUSED = 0
+
+
+def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True):
+    f = kq.lib()["_ZN2kq10int4_routeEjjjjbbiPNS_6skinny4PlanE"]
+    f.restype = C.c_int
+    return f(*(C.c_uint32(a) for a in (M, K, G, batch)), C.c_bool(inter), C.c_bool(meta8),
+             C.c_int(path), None)
+
+
+# AUTO's choice where the skinny kernels were slower than the path they had
+# replaced (measured by 6% to 44%), and where they are the faster one.
+@pytest.mark.parametrize("M,K,G,batch,inter,want", [
+    (8192, 28672, 32, 2, True, VALU), (13824, 5120, 32, 2, True, VALU),
+    (23570, 18784, 32, 3, True, VALU), (6912, 1792, 32, 3, True, VALU),
+    (18816, 2048, 64, 16, False, MFMA), (20138, 2688, 64, 13, False, MFMA),
+    (18598, 2944, 64, 13, True, MFMA), (14336, 4096, 64, 16, False, MFMA),
+    (20361, 1024, 64, 11, False, MFMA), (24570, 640, 64, 15, True, MFMA),
+    (7089, 6144, 64, 11, True, MFMA), (14336, 4096, 64, 8, True, MFMA),
+    (28672, 8192, 64, 8, True, MFMA), (28672, 8192, 128, 16, False, MFMA),
+    (4096, 4096, 64, 8, True, SKINNY), (1024, 4096, 64, 8, True, SKINNY),
+    (4096, 14336, 64, 8, True, SKINNY), (8192, 28672, 128, 16, False, SKINNY),
+    (4096, 24448, 64, 8, True, SKINNY), (18205, 3456, 64, 7, False, SKINNY),
+    (5003, 2848, 32, 4, True, SKINNY), (2880, 5024, 32, 4, True, SKINNY),
+    (4096, 4096, 64, 1, True, VALU), (1024, 4096, 64, 2, True, VALU),
+])
+def test_int4_auto_route(M, K, G, batch, inter, want):
+    assert int4_route(M, K, G, batch, inter) == want
+
+
 # Standalone gate/up: the streaming (2 tokens) or per-tile kernel where the
 # partitioned kernel's plan and staging of every token's x cost more than it
 # saves (measured 1.1 to 1.56 times as long on the False rows).
