@@ -45,7 +45,10 @@ typedef enum kq_dtype { KQ_F16 = 0, KQ_BF16 = 1, KQ_F32 = 2 } kq_dtype;
  * KQ_PATH_SCALAR: the debug scalar kernel, one thread per (row, token) with
  * a plain per-chunk loop and no staging, after gemv_int4_scalar (v0,
  * int4-gemv/src/kernels.metal:71-95) -- slow, for checking the fast paths
- * on the device; AUTO never picks it. */
+ * on the device; AUTO never picks it.
+ * KQ_PATH_MFMA: the matrix cores, G <= 128 with K % 128 == 0 (separate scales and
+ * biases 8-byte aligned); separate ones with G = 128 and K / 128 odd, K >= 256,
+ * run the skinny matrix-core kernels instead of int4_mfma. */
 typedef enum kq_int4_path {
     KQ_PATH_AUTO = 0,
     KQ_PATH_VALU = 1,
@@ -102,6 +105,7 @@ kq_status kq_int4_gemv_path(const uint32_t* W, const void* S, const void* B, kq_
  * MFMA: rows = K parts P per workgroup (a divisor of K/128; at most 8 with
  * 2 or 4 tiles per wave, else 16), unroll = 10 * T + D with T the 16-row
  * tiles per wave and D its ring depth in steps: 12, 24 or 42.
+ * The launch shape given is the one that runs.
  * Returns KQ_EUNSUPPORTED for a shape the family cannot run. Used by the
  * benchmark sweeps and the tests. */
 kq_status kq_int4_gemv_cfg(const uint32_t* W, const void* S, const void* B, kq_dtype sb_dtype,

@@ -69,18 +69,17 @@ int choose_int4(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, 
     // time a call)
     if (path == KQ_PATH_AUTO && batch == 1 && valu_ok) path = KQ_PATH_VALU;
     if (path == KQ_PATH_VALU) return valu_ok ? path : KQ_PATH_AUTO;
-    // the matrix-core path reads a span's separate scales / biases as one
-    // 4- or 8-byte word each, at 128-wide groups also the word of the last row's
-    // last two spans: with an odd number of spans that word would end past the
-    // array, and the range check would zero it
-    const bool mfma_shape = (inter || meta8) && kq::int4_mfma_plan(M, K, G, batch, cfg, p.mp);
-    const bool mfma_ok = mfma_shape && (inter || G != 128 || (K / 128) % 2 == 0);
-    // ... those go to the skinny kernels where the matrix cores are asked for, or
-    // the only path that takes K
-    if (mfma_shape && !mfma_ok && (path == KQ_PATH_MFMA || !valu_ok) &&
-        kq::int4_skinny_plan(M, K, G, batch, inter, p.sp))
-        return kq::kPathSkinny;
-    if (path == KQ_PATH_MFMA) return mfma_ok ? path : KQ_PATH_AUTO;
+    // int4_mfma reads a span's separate scales / biases as one 4- or 8-byte word
+    // each; an odd number of 128-wide groups takes 2-byte loads there, and the skinny
+    // kernels, ten times as exact, take those calls where they can (not K = 128:
+    // 8616 rows, 13 tokens int4_mfma 5.8, vector 27.5 us)
+    const bool mfma_ok = (inter || meta8) && kq::int4_mfma_plan(M, K, G, batch, cfg, p.mp);
+    const bool odd = !inter && G == 128 && (K / 128) % 2 != 0;
+    auto mfma_path = [&] {
+        return odd && !forced && kq::int4_skinny_plan(M, K, G, batch, inter, p.sp) ? kq::kPathSkinny
+                                                                                  : (int)KQ_PATH_MFMA;
+    };
+    if (path == KQ_PATH_MFMA) return mfma_ok ? mfma_path() : (int)KQ_PATH_AUTO;
     if (!valu_ok && !mfma_ok) return KQ_PATH_AUTO;
     // Crossover, in batch-1 vector passes: a vector pass takes up to 4 tokens
     // (int4_valu_cost), a matrix-core pass all of them at ~1.2 (29.3-30.3 us
@@ -107,7 +106,7 @@ int choose_int4(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, 
             (path == KQ_PATH_MFMA ? 0.95 * kq::int4_mfma_pass_us(p.mp, G, batch)
                                   : kq::int4_valu_pass_us(p.vp, M, K, G)))
         return kq::kPathSkinny;
-    return path;
+    return path == KQ_PATH_MFMA ? mfma_path() : path;
 }
 
 kq_status run_int4(const uint32_t* W, const void* S, const void* B, kq_dtype sb_dtype,
@@ -192,9 +191,9 @@ uint32_t cu_count() {
 
 namespace kq {
 int int4_route(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, bool meta8, int path,
-               skinny::Plan* sp) {
+               skinny::Plan* sp, const Int4Cfg* forced) {
     Int4Plans p;
-    const int r = choose_int4(M, K, G, batch, inter, meta8, path, nullptr, p);
+    const int r = choose_int4(M, K, G, batch, inter, meta8, path, forced, p);
     if (sp && r == kPathSkinny) *sp = p.sp;
     return r;
 }

@@ -280,9 +280,18 @@ struct MWin<4, false> {
     u32x4 s, b;  // 2 spans x 4 halves
 };
 
-template <int NG, bool SB>
+// ODD: an odd number of spans of one 2-byte value each. The word of the last row's
+// last two spans would end past the array, and the range check would zero it,
+// so the values are loaded one by one.
+template <int NG, bool SB, bool ODD>
 __device__ __forceinline__ void load_mwin(MWin<NG, SB>& m, rsrc_t rs, rsrc_t rb, uint32_t vo) {
-    if constexpr (SB) {
+    if constexpr (ODD) {
+        static_assert(NG == 1 && !SB, "a span's values fill whole words in every other layout");
+        m.s = __builtin_amdgcn_raw_buffer_load_b16(rs, vo, 0, 0) |
+              (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs, vo + 2, 0, 0) << 16;
+        m.b = __builtin_amdgcn_raw_buffer_load_b16(rb, vo, 0, 0) |
+              (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rb, vo + 2, 0, 0) << 16;
+    } else if constexpr (SB) {
         if constexpr (NG == 1) m.a = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, 0, 0);
         else if constexpr (NG == 2) m.a = __builtin_amdgcn_raw_buffer_load_b128(rs, vo, 0, 0);
         else {
@@ -350,7 +359,7 @@ __device__ __forceinline__ void static_for(Fn&& f) {
     }
 }
 
-template <int GM, bool SB, bool BF, int T, int WAVES>
+template <int GM, bool SB, bool BF, int T, int WAVES, bool ODD>
 __global__ __launch_bounds__(64 * WAVES) void int4_mfma(Args A) {
     constexpr int NG = 128 / GM;         // quant groups per span
     constexpr int NP = (NG + 1) / 2;     // group pairs (correction MFMAs) per span
@@ -448,8 +457,8 @@ __global__ __launch_bounds__(64 * WAVES) void int4_mfma(Args A) {
             const uint32_t lspan = p * A.J + (j2 < A.J ? j2 : A.J - 1);
 #pragma unroll
             for (int i = 0; i < T; ++i)
-                load_mwin<NG, SB>(mwb[i], rS, rB,
-                                  mvo[i] + lspan * NG * MB + (lok ? 0u : kOOB));
+                load_mwin<NG, SB, ODD>(mwb[i], rS, rB,
+                                       mvo[i] + lspan * NG * MB + (lok ? 0u : kOOB));
         }
         if constexpr (std::is_same_v<std::decay_t<decltype(e)>, SlotE<T>>) {
             // the pair (span, span + 1); its offset goes in the lane offset, so
@@ -623,9 +632,9 @@ __global__ __launch_bounds__(64 * WAVES) void int4_mfma(Args A) {
     });
 }
 
-template <int GM, bool SB, bool BF, int T, int WAVES>
+template <int GM, bool SB, bool BF, int T, int WAVES, bool ODD>
 hipError_t go(const Args& a, const Plan& pl, hipStream_t s) {
-    auto kern = int4_mfma<GM, SB, BF, T, WAVES>;
+    auto kern = int4_mfma<GM, SB, BF, T, WAVES, ODD>;
     if (pl.lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -636,11 +645,13 @@ hipError_t go(const Args& a, const Plan& pl, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int GM, bool SB, bool BF>
+template <int GM, bool SB, bool BF, bool ODD = false>
 hipError_t go_td(const Args& a, const Plan& pl, hipStream_t s) {
-    if (pl.T == 4) return go<GM, SB, BF, 4, max_waves(GM, 4)>(a, pl, s);
-    if (pl.T == 2) return go<GM, SB, BF, 2, max_waves(GM, 2)>(a, pl, s);
-    if (pl.T == 1) return go<GM, SB, BF, 1, max_waves(GM, 1)>(a, pl, s);
+    if constexpr (GM == 128 && !SB && !ODD)
+        if (a.gpr & 1) return go_td<GM, SB, BF, true>(a, pl, s);
+    if (pl.T == 4) return go<GM, SB, BF, 4, max_waves(GM, 4), ODD>(a, pl, s);
+    if (pl.T == 2) return go<GM, SB, BF, 2, max_waves(GM, 2), ODD>(a, pl, s);
+    if (pl.T == 1) return go<GM, SB, BF, 1, max_waves(GM, 1), ODD>(a, pl, s);
     return hipErrorInvalidValue;
 }
 

@@ -91,12 +91,12 @@ hipError_t launch_vq_skinny(const uint8_t* IDX, const uint16_t* C, const uint16_
                             void* Y, bool y_f32, uint32_t M, uint32_t K, uint32_t rows_per_cb,
                             uint32_t scale_group, uint32_t batch, const skinny::Plan& pl, hipStream_t s);
 
-// The path an int4 call takes without a forced launch shape: KQ_PATH_*, or
+// The path an int4 call takes (forced: a launch shape, or null): KQ_PATH_*, or
 // kPathSkinny (its plan to sp, if given), KQ_PATH_AUTO where it is refused. meta8:
 // scales and biases start at multiples of 8 bytes.
 constexpr int kPathSkinny = 4;
 int int4_route(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, bool meta8, int path,
-               skinny::Plan* sp);
+               skinny::Plan* sp, const Int4Cfg* forced);
 
 // Debug scalar path: one thread per (row, token), plain chunk loop (v0).
 hipError_t launch_int4_scalar(const uint32_t* W, const uint16_t* S, const uint16_t* B,

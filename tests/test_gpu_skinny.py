@@ -114,6 +114,24 @@ def test_odd_spans_split_g128(gpu, M, K, path):
         assert inf_rel(to_f64(y), ref) < 1e-5, f"{M}x{K} b{batch}"
 
 
+# The same in int4_mfma: K too short for the skinny kernels, and its launch shape
+# given (P, 10 T + ring depth; none divides its spans evenly into windows). The last
+# row's last scale, and its bias, are the last two bytes of their arrays. 5e-5 of
+# the largest value: sums of products that carry 64 and 1024 + q are up to 1.4e-5 off.
+@pytest.mark.parametrize("M,K,parts,unroll", [(300, 128, 0, 0), (17, 128, 1, 42), (300, 1152, 1, 12), (257, 1152, 9, 12),
+                                              (300, 1152, 3, 24), (4097, 1152, 3, 42)])
+def test_odd_spans_split_g128_int4_mfma(gpu, M, K, parts, unroll):
+    for batch in (1, 5, 16):
+        p = gen.int4_problem(M, K, 128, batch=batch, seed=K + batch + parts)
+        y = torch.full((batch, M), float("nan"), dtype=torch.float32, device=gpu)
+        kq.int4_gemv(dev(p["W"], gpu), dev(p["S"], gpu), dev(p["X"], gpu), y, kq.GemvParams(M, K, 128),
+                     B=dev(p["B"], gpu), batch=batch, path=kq.PATH_MFMA, rows=parts, unroll=unroll)
+        torch.cuda.synchronize()
+        ref = oracle.int4_gemv(p["W"], p["S"], p["B"], p["X"], M, K, 128, False, oracle.F16)
+        assert inf_rel(to_f64(y), ref) < 5e-5, f"{M}x{K} P{parts} T,D {unroll} b{batch}"
+        assert inf_rel(to_f64(y)[:, -1:], ref[:, -1:]) < 5e-4, "the last row"
+
+
 # Codebook blocks of an odd tile count: the skinny kernels with a workgroup a
 # block, or the passes, whichever the route gives.
 @pytest.mark.parametrize("M,K,rpc,sg", [(5120, 512, 1264, 512), (2768, 1056, 592, 32), (4128, 288, 1376, 288)])

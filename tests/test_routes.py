@@ -32,11 +32,11 @@ VALU, MFMA, SKINNY = kq.PATH_VALU, kq.PATH_MFMA, 4
 REFUSED = 0
 
 
-def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True):
-    f = kq.lib()["_ZN2kq10int4_routeEjjjjbbiPNS_6skinny4PlanE"]
+def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True, forced=None):
+    f = kq.lib()["_ZN2kq10int4_routeEjjjjbbiPNS_6skinny4PlanEPKNS_7Int4CfgE"]
     f.restype = C.c_int
     return f(*(C.c_uint32(a) for a in (M, K, G, batch)), C.c_bool(inter), C.c_bool(meta8),
-             C.c_int(path), None)
+             C.c_int(path), None, (C.c_int * 2)(*forced) if forced else None)
 
 
 # AUTO's choice where the skinny kernels were slower than the path they had
@@ -57,6 +57,21 @@ def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True):
 ])
 def test_int4_auto_route(M, K, G, batch, inter, want):
     assert int4_route(M, K, G, batch, inter) == want
+
+
+# Separate 128-wide groups with an odd number of spans: the skinny kernels where
+# the matrix cores are asked for or chosen, int4_mfma where K is too short for them
+# or its launch shape is given.
+def test_int4_odd_spans_route():
+    for batch in (1, 5, 16):
+        assert int4_route(300, 128, 128, batch, False, MFMA) == MFMA
+        assert int4_route(300, 1152, 128, batch, False, MFMA) == SKINNY
+        for forced in ((1, 12), (3, 24), (9, 12), (3, 42)):
+            assert int4_route(300, 1152, 128, batch, False, MFMA, forced=forced) == MFMA
+        assert int4_route(300, 1152, 128, batch, False, MFMA, forced=(2, 12)) == REFUSED
+        assert int4_route(300, 1152, 128, batch, False, MFMA, meta8=False) == REFUSED
+    assert int4_route(640, 13440, 128, 5, False) == SKINNY
+    assert int4_route(300, 128, 128, 16, False) == MFMA
 
 
 # Standalone gate/up: the streaming (2 tokens) or per-tile kernel where the
