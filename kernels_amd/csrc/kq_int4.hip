@@ -529,11 +529,6 @@ double int4_valu_pass_us(const Int4Passes& ps, uint32_t M, uint32_t K, uint32_t 
     return us;
 }
 
-size_t int4_valu_lds_bytes(uint32_t K, uint32_t batch) {
-    const uint32_t nchp = ((K >> 5) + 63) / 64 * 64;
-    return vlds_x(batch < kMaxNB ? batch : kMaxNB, nchp);
-}
-
 bool int4_valu_supported(uint32_t K, Int4Cfg cfg) {
     VPlan pl;
     return make_vplan(16, K, 1, cfg, pl);

@@ -31,7 +31,6 @@ struct Int4Passes {
     uint32_t n;  // 0: no plan
 };
 Int4Passes int4_valu_passes(uint32_t M, uint32_t K, uint32_t batch, Int4Cfg cfg);
-size_t int4_valu_lds_bytes(uint32_t K, uint32_t batch);
 // The passes in batch-1-pass units x 100 (AUTO's crossover).
 uint32_t int4_valu_cost(const Int4Passes& ps);
 // Their modelled duration (us; AUTO's crossovers, with int4_mfma and with the
@@ -117,7 +116,6 @@ hipError_t launch_vq(const uint8_t* IDX, const uint16_t* C, const uint16_t* S, c
 // VQ quantiser (kq_vq_quant.hip)
 size_t vq_quant_ws_bytes(uint32_t M, uint32_t K, uint32_t scale_group, uint32_t rows_per_cb,
                          uint32_t sample);
-uint32_t vq_quant_launches(uint32_t iters);
 hipError_t launch_vq_quantize(const void* W, int w_dtype, uint32_t M, uint32_t K,
                               uint32_t rows_per_cb, uint32_t scale_group, uint32_t iters,
                               uint32_t sample, uint64_t seed, uint8_t* IDX, uint16_t* Cb,

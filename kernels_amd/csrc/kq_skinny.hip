@@ -71,7 +71,6 @@ skinny::Args make_args(const skinny::Plan& pl, uint32_t M, uint32_t K, uint32_t 
     a.Q = pl.Q;
     a.J = pl.J;
     a.NP = pl.NP;
-    a.ntiles = (M + 15) / 16;
     a.tiles_wg = pl.tiles_wg;
     a.rounds = pl.rounds;
     a.part_lds = (uint32_t)pl.part_lds;
@@ -132,7 +131,8 @@ double int4_skinny_us(const skinny::Plan& pl, uint32_t G, uint32_t batch, bool i
 
 bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, skinny::Plan& pl) {
     if (batch < 1 || batch > 16 || !(G == 32 || G == 64 || G == 128) || K % G) return false;
-    if (!inter && G == 32 && batch <= 8) return false;  // its windows spill
+    // not in use: one tile's windows spill there, two tiles alone are unmeasured
+    if (!inter && G == 32 && batch <= 8) return false;
     return make_plan(M, K, batch, int4_tmax(G), even_share(M), 0, pl);
 }
 

@@ -54,7 +54,8 @@ namespace skinny {
 
 constexpr uint32_t kPair = 256;      // k of a step
 constexpr uint32_t kWin = 4;         // steps of a scale window
-// Waves a workgroup: one tile a wave fits 128 VGPRs (16 waves, 4 a SIMD).
+// Waves a workgroup: one tile a wave and up to 8 tokens leave room for 16 waves (4 a
+// SIMD, 128 VGPRs: 106-128 in use, 7 spilled with 64-wide groups' separate scales).
 __host__ __device__ constexpr uint32_t max_waves(uint32_t T, bool x8) { return T == 1 && x8 ? 16 : 8; }
 
 struct Args {
@@ -68,7 +69,7 @@ struct Args {
     uint32_t gpr;        // scale groups per row
     uint32_t gshift;     // KIND 1, groups of 128 or more: log2 of the group
     uint32_t P, Q, J, NP;  // K parts, row lanes, pairs per part, pairs per row
-    uint32_t ntiles, tiles_wg, rounds;
+    uint32_t tiles_wg, rounds;
     uint32_t rpc, cb_lds;  // KIND 1: rows per codebook (multiple of 16), LDS bytes of the copies
     uint32_t part_lds;     // LDS bytes of the K-part sums (the x stages follow)
 };
@@ -113,12 +114,12 @@ __device__ __forceinline__ u32x4 xorder(u32x4 v) {
 __device__ __forceinline__ uint32_t lds_word(uint32_t addr) {
     return *(const __attribute__((address_space(3))) uint32_t*)(uintptr_t)addr;
 }
-// The codewords of a word's 4 indices; cbase = (block << 16) | (lane << 2).
-__device__ __forceinline__ f16x8 codewords(uint32_t w, uint32_t cbase) {
-    const u32x4 v{lds_word(__builtin_amdgcn_perm(w, cbase, 0x0C020400u)),
-                  lds_word(__builtin_amdgcn_perm(w, cbase, 0x0C020500u)),
-                  lds_word(__builtin_amdgcn_perm(w, cbase, 0x0C020600u)),
-                  lds_word(__builtin_amdgcn_perm(w, cbase, 0x0C020700u))};
+// The codewords of a word's 4 indices, from the lane's copies (lane4 = lane << 2).
+__device__ __forceinline__ f16x8 codewords(uint32_t w, uint32_t lane4) {
+    const u32x4 v{lds_word(__builtin_amdgcn_perm(w, lane4, 0x0C0C0400u)),
+                  lds_word(__builtin_amdgcn_perm(w, lane4, 0x0C0C0500u)),
+                  lds_word(__builtin_amdgcn_perm(w, lane4, 0x0C0C0600u)),
+                  lds_word(__builtin_amdgcn_perm(w, lane4, 0x0C0C0700u))};
     return __builtin_bit_cast(f16x8, v);
 }
 
@@ -158,17 +159,11 @@ __global__ __launch_bounds__(64 * max_waves(T, X8)) void skinny_k(Args A) {
     const rsrc_t rB = make_rsrc(reinterpret_cast<const uint8_t*>(KIND == 0 && !SB ? A.B : A.S) +
                                     (size_t)row0 * srowb, rows * srowb);
 
-    // codebook blocks of the workgroup's rows (at most 2)
-    u32x4 cbq[2];
-    uint32_t cb0 = 0, ncb = 0;
-    if constexpr (KIND == 1) {
-        cb0 = row0 / A.rpc;
-        ncb = (row0 + rows - 1) / A.rpc - cb0 + 1;
-        const rsrc_t rC = make_rsrc(A.C + (size_t)cb0 * 512, ncb * 1024);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-            cbq[b] = __builtin_amdgcn_raw_buffer_load_b128(rC, lane * 16 + b * 1024u, 0, 0);
-    }
+    // the codebook of the workgroup's rows
+    u32x4 cbq{0, 0, 0, 0};
+    if constexpr (KIND == 1)
+        cbq = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(A.C + (size_t)(row0 / A.rpc) * 512, 1024),
+                                                    lane * 16, 0, 0);
 
     // lane parts of the addresses
     // x load j: the pair's 256 k of tokens 2j, 2j + 1 (512 bytes each)
@@ -284,20 +279,15 @@ __global__ __launch_bounds__(64 * max_waves(T, X8)) void skinny_k(Args A) {
     });
 
     if constexpr (KIND == 1) {
-        // 64 copies of every entry, entry e of block b at (b << 16) | (e << 8):
-        // wave w stores copy groups (w' + lane) % 16, w' = w, w + waves, ..., of
-        // the lane's 4 entries (conflict-free)
+        // 64 copies of every entry, entry e at e << 8: wave w stores copy groups
+        // (w' + lane) % 16, w' = w, w + waves, ..., of the lane's 4 entries
+        // (conflict-free)
+        unsigned char* eb = smem + lane * 1024;
+        for (uint32_t w2 = wave; w2 < 16; w2 += nthr >> 6) {
+            const uint32_t g = (w2 + lane) & 15;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            if (b >= (int)ncb) break;  // uniform
-            unsigned char* eb = smem + (uint32_t)b * 65536 + lane * 1024;
-            for (uint32_t w2 = wave; w2 < 16; w2 += nthr >> 6) {
-                const uint32_t g = (w2 + lane) & 15;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    *reinterpret_cast<u32x4*>(eb + k * 256 + g * 16) =
-                        u32x4{cbq[b][k], cbq[b][k], cbq[b][k], cbq[b][k]};
-            }
+            for (int k = 0; k < 4; ++k)
+                *reinterpret_cast<u32x4*>(eb + k * 256 + g * 16) = u32x4{cbq[k], cbq[k], cbq[k], cbq[k]};
         }
         __syncthreads();
     }
@@ -371,18 +361,12 @@ __global__ __launch_bounds__(64 * max_waves(T, X8)) void skinny_k(Args A) {
             // x to the wave's LDS (chunk c of token t at c ^ t), back as operands
 #pragma unroll
             for (int j = 0; j < NX; ++j) *reinterpret_cast<u32x4*>(xst + xwo[j]) = xorder<KIND>(e.x[j]);
-            uint32_t cbase[T], m[T][MR ? MR : 1];
+            uint32_t m[T][MR ? MR : 1];
 #pragma unroll
-            for (int i = 0; i < T; ++i) {
+            for (int i = 0; i < T; ++i)
 #pragma unroll
                 for (int z = 0; z < MR && !SB; ++z)
                     m[i][z] = mfma::bperm(4 * (n + 16 * (c.j % kWin)), mw[i][z]);
-                cbase[i] = 0;
-                if constexpr (KIND == 1) {
-                    const uint32_t row = min(row0 + (tile_of(c.round) + i) * 16, M - 1);
-                    cbase[i] = (__builtin_amdgcn_readfirstlane(row / A.rpc - cb0) << 16) | (lane << 2);
-                }
-            }
             // KIND 1: products of at most 64 k in a chain, and the step's sums
             // apart from the running ones: the vector path's error, 1e-7 (one
             // chain of all of a wave's k: 4.1e-7 at K = 28672)
@@ -412,7 +396,7 @@ __global__ __launch_bounds__(64 * max_waves(T, X8)) void skinny_k(Args A) {
                     f32x4 dg[NC];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const f16x8 b = KIND == 0 ? dq64(w[j], kc) : codewords(w[j], cbase[i]);
+                        const f16x8 b = KIND == 0 ? dq64(w[j], kc) : codewords(w[j], lane << 2);
                         dg[j / PERC] = mfma::mma16(xa[j], b, j % PERC == 0 ? zero : dg[j / PERC]);
                     }
 #pragma unroll
@@ -498,10 +482,15 @@ hipError_t go(const Args& a, const Plan& pl, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Four tiles spill with 8 groups a step.
+// No four tiles with 8 groups a step (no room for their registers), and no separate
+// scales of 8 groups up to 8 tokens (one tile spills 39-49 VGPRs).
 template <int KIND, int GM, bool SB, bool BF>
 hipError_t dispatch(const Args& a, const Plan& pl, hipStream_t s) {
     const bool x8 = a.ntok <= 8;
+    if constexpr (KIND == 0 && GM == 32 && !SB) {
+        if (x8 || pl.T > 2) return hipErrorInvalidValue;
+        return pl.T == 1 ? go<KIND, GM, SB, BF, 1, false>(a, pl, s) : go<KIND, GM, SB, BF, 2, false>(a, pl, s);
+    }
     if (pl.T == 1) return x8 ? go<KIND, GM, SB, BF, 1, true>(a, pl, s) : go<KIND, GM, SB, BF, 1, false>(a, pl, s);
     if (pl.T == 2) return x8 ? go<KIND, GM, SB, BF, 2, true>(a, pl, s) : go<KIND, GM, SB, BF, 2, false>(a, pl, s);
     if constexpr (GM != 32)

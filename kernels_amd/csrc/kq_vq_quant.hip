@@ -729,8 +729,6 @@ size_t vq_quant_ws_bytes(uint32_t M, uint32_t K, uint32_t scale_group, uint32_t 
     return qws_layout(M, K, scale_group, rows_per_cb, sample).total;
 }
 
-uint32_t vq_quant_launches(uint32_t iters) { return 3 + 2 * iters; }
-
 hipError_t launch_vq_quantize(const void* W, int w_dtype, uint32_t M, uint32_t K,
                               uint32_t rows_per_cb, uint32_t scale_group, uint32_t iters,
                               uint32_t sample, uint64_t seed, uint8_t* IDX, uint16_t* Cb,
