@@ -77,7 +77,12 @@ skinny::Args make_args(const skinny::Plan& pl, uint32_t M, uint32_t K, uint32_t 
     return a;
 }
 
-uint32_t int4_tmax(uint32_t G) { return G == 32 ? 2 : 4; }
+// Four tiles of 64-wide groups' separate scales spill above 8 tokens: two instead
+// take 0.68-1.10 times as long, 0.84 on average of 150 calls (10888x2048, 10 tokens:
+// 11.9 -> 8.1 us).
+uint32_t int4_tmax(uint32_t G, uint32_t batch, bool inter) {
+    return G == 32 || (G == 64 && !inter && batch > 8) ? 2 : 4;
+}
 
 // Tiles a workgroup: every CU's share.
 uint32_t even_share(uint32_t M) {
@@ -119,12 +124,11 @@ static double skinny_us(const skinny::Plan& pl, uint32_t batch, double form) {
 }
 
 // A step's cost by int4 layout (medians of 14000 calls, nine in ten within 15%): 8
-// groups a pair take more work for scales, four tiles of 64-wide groups' separate
-// scales spill.
+// groups a pair take more work for scales.
 double int4_skinny_us(const skinny::Plan& pl, uint32_t G, uint32_t batch, bool inter) {
     const bool two8 = inter && pl.T == 2 && batch <= 8;
     double form = two8 ? 0.98 : 0.92;
-    if (G == 64) form = pl.T < 4 ? (two8 ? 1.07 : 1.03) : inter ? 1.1 : 1.6;
+    if (G == 64) form = pl.T == 4 ? 1.1 : two8 ? 1.07 : 1.03;
     if (G == 32) form = !inter ? 1.08 : two8 ? 1.45 : 1.22;
     return skinny_us(pl, batch, form) + (pl.T > 1 ? 0.3 : 0.0);
 }
@@ -133,7 +137,7 @@ bool int4_skinny_plan(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool i
     if (batch < 1 || batch > 16 || !(G == 32 || G == 64 || G == 128) || K % G) return false;
     // not in use: one tile's windows spill there, two tiles alone are unmeasured
     if (!inter && G == 32 && batch <= 8) return false;
-    return make_plan(M, K, batch, int4_tmax(G), even_share(M), 0, pl);
+    return make_plan(M, K, batch, int4_tmax(G, batch, inter), even_share(M), 0, pl);
 }
 
 hipError_t launch_int4_skinny(const uint32_t* W, const uint16_t* S, const uint16_t* B, int meta_kind,

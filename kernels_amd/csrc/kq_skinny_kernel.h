@@ -482,8 +482,9 @@ hipError_t go(const Args& a, const Plan& pl, hipStream_t s) {
     return hipGetLastError();
 }
 
-// No four tiles with 8 groups a step (no room for their registers), and no separate
-// scales of 8 groups up to 8 tokens (one tile spills 39-49 VGPRs).
+// Variants with room for their registers: no four tiles with 8 groups a step, nor
+// with 4 groups' separate scales above 8 tokens (26-58 VGPRs spilled), and no
+// separate scales of 8 groups up to 8 tokens (one tile spills 39-49).
 template <int KIND, int GM, bool SB, bool BF>
 hipError_t dispatch(const Args& a, const Plan& pl, hipStream_t s) {
     const bool x8 = a.ntok <= 8;
@@ -493,7 +494,9 @@ hipError_t dispatch(const Args& a, const Plan& pl, hipStream_t s) {
     }
     if (pl.T == 1) return x8 ? go<KIND, GM, SB, BF, 1, true>(a, pl, s) : go<KIND, GM, SB, BF, 1, false>(a, pl, s);
     if (pl.T == 2) return x8 ? go<KIND, GM, SB, BF, 2, true>(a, pl, s) : go<KIND, GM, SB, BF, 2, false>(a, pl, s);
-    if constexpr (GM != 32)
+    if constexpr (KIND == 0 && GM == 64 && !SB) {
+        if (x8) return go<KIND, GM, SB, BF, 4, true>(a, pl, s);
+    } else if constexpr (GM != 32)
         return x8 ? go<KIND, GM, SB, BF, 4, true>(a, pl, s) : go<KIND, GM, SB, BF, 4, false>(a, pl, s);
     return hipErrorInvalidValue;
 }

@@ -46,13 +46,13 @@ def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True, forced=None
     (23570, 18784, 32, 3, True, VALU), (6912, 1792, 32, 3, True, VALU),
     (18816, 2048, 64, 16, False, MFMA), (20138, 2688, 64, 13, False, MFMA),
     (18598, 2944, 64, 13, True, MFMA), (14336, 4096, 64, 16, False, MFMA),
-    (20361, 1024, 64, 11, False, MFMA), (24570, 640, 64, 15, True, MFMA),
+    (24570, 640, 64, 15, True, MFMA),
     (7089, 6144, 64, 11, True, MFMA), (14336, 4096, 64, 8, True, MFMA),
     (28672, 8192, 64, 8, True, MFMA), (28672, 8192, 128, 16, False, MFMA),
     (4096, 4096, 64, 8, True, SKINNY), (1024, 4096, 64, 8, True, SKINNY),
     (4096, 14336, 64, 8, True, SKINNY), (8192, 28672, 128, 16, False, SKINNY),
     (4096, 24448, 64, 8, True, SKINNY), (18205, 3456, 64, 7, False, SKINNY),
-    (5003, 2848, 32, 4, True, SKINNY), (2880, 5024, 32, 4, True, SKINNY),
+    (20361, 1024, 64, 11, False, SKINNY), (5003, 2848, 32, 4, True, SKINNY), (2880, 5024, 32, 4, True, SKINNY),
     (4096, 4096, 64, 1, True, VALU), (1024, 4096, 64, 2, True, VALU),
 ])
 def test_int4_auto_route(M, K, G, batch, inter, want):
