@@ -228,8 +228,8 @@ void kq_moe_default_desc(kq_moe_desc* d);
 /* Bytes of workspace the MoE entry points need for `batch` tokens: the router
  * logits, a completion counter, the one-launch block's grid-barrier word, the
  * routing plan (distinct experts and their token slots) that the block's
- * gate/up and down kernels read, and the per-slot down products of the block
- * at 6 or more tokens. A new workspace must be zeroed once with
+ * gate/up and down kernels read, and the per-slot down products (from as many
+ * tokens as the shape gives: 6 at the gpt-oss-120b shapes). A new workspace must be zeroed once with
  * kq_moe_workspace_init (a kernel, not a memset, so it can sit in a captured
  * graph) before its first use; every call leaves it ready for the next.
  * Calls sharing one workspace must be stream-ordered. The uint32 at byte
@@ -278,8 +278,8 @@ kq_status kq_moe_gate_up_swiglu(const uint8_t* pool, const kq_moe_desc* d,
 
 /* Y[b][m] = sum_k wgt[b][k] * (down_e(H[b][k])[m] + BId[m]), e = idx[b][k],
  * summed in k order. Y: [batch][hidden] of y_dtype (KQ_F32 or KQ_F16).
- * A workspace (optional) may take the per-slot products (6 or more tokens), so
- * it must not be in use by work on another stream.
+ * A workspace is optional; where one is given the call may write it, at any
+ * batch (the per-slot products), so calls that share one must be stream-ordered.
  * Replaces: fused_down_combine moe-fused/src/kernels.metal:224-265
  *   (encoded at moe-fused/src/main.mm:196-204). */
 kq_status kq_moe_down_combine(const uint8_t* pool, const kq_moe_desc* d,
@@ -288,7 +288,8 @@ kq_status kq_moe_down_combine(const uint8_t* pool, const kq_moe_desc* d,
                               void* ws, size_t ws_bytes, kq_stream_t stream);
 
 /* The three passes back to back on one stream (encodeFused,
- * moe-fused/src/main.mm:176-206): three launches; from 6 tokens down writes
+ * moe-fused/src/main.mm:176-206): three launches; where the slots' h vectors
+ * don't fit one workgroup (from 6 tokens at the gpt-oss-120b shapes) down writes
  * per-slot products to the workspace and a fourth, small launch sums them in
  * slot order. idx, wgt, xh (if X is fp32) and H are caller-provided
  * outputs/intermediates of the sizes above. */

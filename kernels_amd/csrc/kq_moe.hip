@@ -25,9 +25,9 @@
 //      item's loads; the activations are prepared once per workgroup in LDS
 //      (at one token, held in registers); down keeps per-slot
 //      wgt * (down . h + bias) in LDS and sums the slots in k order;
-//    - expert-partitioned (the block's gate/up from 3 tokens, moe_gu_part_k;
-//      its down from 6 tokens, moe_dn_part_k): one round of one workgroup
-//      per CU; each plan entry gets workgroups in proportion to its cost
+//    - expert-partitioned (the block's gate/up from 2 tokens, moe_gu_part_k;
+//      its down past the streaming form's limit, moe_dn_part_k): one round of
+//      one workgroup per CU; each plan entry gets workgroups in proportion to its cost
 //      (rows x (4 + 3 x slots)), and a workgroup streams a row chunk of one
 //      expert with only that expert's activations in LDS; down writes
 //      per-slot products to the workspace and a small moe_combine_k launch
@@ -1784,8 +1784,8 @@ __global__ __launch_bounds__(64 * kStWaves) void moe_gu_part_k(
     else run(std::false_type{});
 }
 
-// Down + weighted products, partitioned by expert (from 6 tokens, where the
-// slots' h vectors no longer fit one workgroup's LDS): workgroup b streams
+// Down + weighted products, partitioned by expert (from 6 tokens at gpt-oss
+// shapes, where the slots' h vectors no longer fit one workgroup's LDS): workgroup b streams
 // the row-pair chunk part_assign gives it of one plan entry's expert with
 // only that expert's h vectors in LDS (one per slot that chose it, at most
 // one per token), and writes wgt_s * (down . h_s + bias) for each of those
