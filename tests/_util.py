@@ -1,4 +1,7 @@
-"""Shared helpers for the tests (device upload, tolerance checks)."""
+"""Shared helpers for the tests (device upload, tolerance checks, the planners'
+choices)."""
+import ctypes as C
+
 import numpy as np
 
 # Tolerance for fp16/fp32 outputs with fp32 accumulation, read as allclose:
@@ -67,3 +70,46 @@ def tie_weights(M, K, seed):
     W += (rng.random((M, K)) < 0.3).astype(np.float32) * np.float32(2.0**-24)
     W[:, :2] = 1.0
     return W
+
+
+# ---- which kernels a call runs, and how: libkq's own C++ functions, declared in
+# kernels_amd/csrc/kq_internal.h (256 compute units are assumed without a GPU)
+class SkinnyPlan(C.Structure):
+    """kq::skinny::Plan: T tiles a wave, P K parts x Q row lanes, J pairs of spans
+    a part, rounds a workgroup."""
+    _fields_ = ([(n, C.c_uint32) for n in ("T", "P", "Q", "J", "NP", "rounds", "tiles_wg", "nwg")] +
+                [(n, C.c_size_t) for n in ("part_lds", "x_lds")])
+
+
+SKINNY, REFUSED = 4, 0  # int4_route beside kq.PATH_VALU, _MFMA and _SCALAR
+
+
+def _internal(name, restype):
+    from kernels_amd import kq
+    f = kq.lib()[name]
+    f.restype = restype
+    return f
+
+
+def int4_route(M, K, G, batch, inter, path=0, meta8=True, forced=None, plan=None):
+    """The path of an int4 call; a SkinnyPlan given as plan is filled for SKINNY."""
+    f = _internal("_ZN2kq10int4_routeEjjjjbbiPNS_6skinny4PlanEPKNS_7Int4CfgE", C.c_int)
+    return f(*(C.c_uint32(a) for a in (M, K, G, batch)), C.c_bool(inter), C.c_bool(meta8), C.c_int(path),
+             C.byref(plan) if plan else None, (C.c_int * 2)(*forced) if forced else None)
+
+
+def vq_takes_skinny(M, K, rpc, sg, batch):
+    f = _internal("_ZN2kq15vq_takes_skinnyEjjjjj", C.c_bool)
+    return f(*(C.c_uint32(a) for a in (M, K, rpc, sg, batch)))
+
+
+def vq_skinny_plan(M, K, rpc, sg, batch):
+    f = _internal("_ZN2kq14vq_skinny_planEjjjjjRNS_6skinny4PlanE", C.c_bool)
+    p = SkinnyPlan()
+    assert f(*(C.c_uint32(a) for a in (M, K, rpc, sg, batch)), C.byref(p))
+    return p
+
+
+def moe_gate_up_partitions(d, batch):
+    f = _internal("_ZN2kq22moe_gate_up_partitionsERK11kq_moe_descj", C.c_bool)
+    return f(C.byref(d), C.c_uint32(batch))

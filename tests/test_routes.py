@@ -1,17 +1,10 @@
-"""Which kernels a call runs, on the CPU: the planners' choices need no GPU (256
-compute units are assumed without one). The functions are libkq's own C++ ones,
-declared in kernels_amd/csrc/kq_internal.h."""
-import ctypes as C
-
+"""Which kernels a call runs, on the CPU: the planners' choices need no GPU."""
 import pytest
 
 from kernels_amd import kq
+from tests._util import REFUSED, SKINNY, int4_route, moe_gate_up_partitions, vq_takes_skinny
 
-
-def vq_takes_skinny(*args):
-    f = kq.lib()["_ZN2kq15vq_takes_skinnyEjjjjj"]
-    f.restype = C.c_bool
-    return f(*(C.c_uint32(a) for a in args))
+VALU, MFMA = kq.PATH_VALU, kq.PATH_MFMA
 
 
 # Codebook blocks whose tiles divide badly would leave the skinny kernels 5-32
@@ -26,17 +19,6 @@ def test_vq_route_follows_the_plans_duration(M, K, rpc, skinny):
     for sg in (32, K):
         for batch in (3, 5, 8, 16):
             assert vq_takes_skinny(M, K, rpc, sg, batch) == skinny, (sg, batch)
-
-
-VALU, MFMA, SKINNY = kq.PATH_VALU, kq.PATH_MFMA, 4
-REFUSED = 0
-
-
-def int4_route(M, K, G, batch, inter, path=kq.PATH_AUTO, meta8=True, forced=None):
-    f = kq.lib()["_ZN2kq10int4_routeEjjjjbbiPNS_6skinny4PlanEPKNS_7Int4CfgE"]
-    f.restype = C.c_int
-    return f(*(C.c_uint32(a) for a in (M, K, G, batch)), C.c_bool(inter), C.c_bool(meta8),
-             C.c_int(path), None, (C.c_int * 2)(*forced) if forced else None)
 
 
 # AUTO's choice where the skinny kernels were slower than the path they had
@@ -85,6 +67,4 @@ def test_int4_odd_spans_route():
 ])
 def test_standalone_gate_up_route(hidden, inter, ne, tk, batch, part):
     d = kq.MoEDesc(hidden=hidden, inter=inter, n_experts=ne, top_k=tk, blob=1 << 25)
-    f = kq.lib()["_ZN2kq22moe_gate_up_partitionsERK11kq_moe_descj"]
-    f.restype = C.c_bool
-    assert f(C.byref(d), C.c_uint32(batch)) == part
+    assert moe_gate_up_partitions(d, batch) == part
