@@ -69,10 +69,10 @@ int choose_int4(uint32_t M, uint32_t K, uint32_t G, uint32_t batch, bool inter, 
     // time a call)
     if (path == KQ_PATH_AUTO && batch == 1 && valu_ok) path = KQ_PATH_VALU;
     if (path == KQ_PATH_VALU) return valu_ok ? path : KQ_PATH_AUTO;
-    // int4_mfma reads a span's separate scales / biases as one 4- or 8-byte word
-    // each; an odd number of 128-wide groups takes 2-byte loads there, and the skinny
-    // kernels, ten times as exact, take those calls where they can (not K = 128:
-    // 8616 rows, 13 tokens int4_mfma 5.8, vector 27.5 us)
+    // int4_mfma reads separate scales / biases as 4- or 8-byte words (two spans' of
+    // 128-wide groups, one by one where a K part has an odd number of them); an odd
+    // number of 128-wide groups goes to the skinny kernels, ten times as exact, where
+    // they can take it (not K = 128: 8616 rows, 13 tokens int4_mfma 5.8, vector 27.5 us)
     const bool mfma_ok = (inter || meta8) && kq::int4_mfma_plan(M, K, G, batch, cfg, p.mp);
     const bool odd = !inter && G == 128 && (K / 128) % 2 != 0;
     auto mfma_path = [&] {

@@ -280,9 +280,9 @@ struct MWin<4, false> {
     u32x4 s, b;  // 2 spans x 4 halves
 };
 
-// ODD: an odd number of spans of one 2-byte value each. The word of the last row's
-// last two spans would end past the array, and the range check would zero it,
-// so the values are loaded one by one.
+// ODD: K parts of an odd number of spans, of one 2-byte value each. The word that
+// begins with the last part's last span would end past the array in the last row,
+// and the range check would zero it, so the values are loaded one by one.
 template <int NG, bool SB, bool ODD>
 __device__ __forceinline__ void load_mwin(MWin<NG, SB>& m, rsrc_t rs, rsrc_t rb, uint32_t vo) {
     if constexpr (ODD) {
@@ -648,7 +648,7 @@ hipError_t go(const Args& a, const Plan& pl, hipStream_t s) {
 template <int GM, bool SB, bool BF, bool ODD = false>
 hipError_t go_td(const Args& a, const Plan& pl, hipStream_t s) {
     if constexpr (GM == 128 && !SB && !ODD)
-        if (a.gpr & 1) return go_td<GM, SB, BF, true>(a, pl, s);
+        if (pl.J & 1) return go_td<GM, SB, BF, true>(a, pl, s);
     if (pl.T == 4) return go<GM, SB, BF, 4, max_waves(GM, 4), ODD>(a, pl, s);
     if (pl.T == 2) return go<GM, SB, BF, 2, max_waves(GM, 2), ODD>(a, pl, s);
     if (pl.T == 1) return go<GM, SB, BF, 1, max_waves(GM, 1), ODD>(a, pl, s);

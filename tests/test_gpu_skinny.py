@@ -217,12 +217,16 @@ def test_odd_spans_split_g128(gpu, M, K, path):
         assert inf_rel(to_f64(y), ref) < 1e-5, f"{M}x{K} b{batch}"
 
 
-# The same in int4_mfma: K too short for the skinny kernels, and its launch shape
-# given (P, 10 T + ring depth; none divides its spans evenly into windows). The last
-# row's last scale, and its bias, are the last two bytes of their arrays. 5e-5 of
-# the largest value: sums of products that carry 64 and 1024 + q are up to 1.4e-5 off.
+# The same in int4_mfma, wherever a K part has an odd number of spans: K too short
+# for the skinny kernels, the launch shape given (P, 10 T + ring depth), and an even
+# number of spans cut into odd parts, by a given P or the planner's (512 and 2048 at
+# few rows). The last row's last scale, and its bias, are the last two bytes of
+# their arrays. 5e-5 of the largest value: sums of products that carry 64 and 1024 +
+# q are up to 1.4e-5 off.
 @pytest.mark.parametrize("M,K,parts,unroll", [(300, 128, 0, 0), (17, 128, 1, 42), (300, 1152, 1, 12), (257, 1152, 9, 12),
-                                              (300, 1152, 3, 24), (4097, 1152, 3, 42)])
+                                              (300, 1152, 3, 24), (4097, 1152, 3, 42), (2, 512, 0, 0),
+                                              (300, 2048, 0, 0), (17, 1536, 4, 12), (17, 1536, 4, 24),
+                                              (300, 256, 2, 42), (100, 14336, 16, 12)])
 def test_odd_spans_split_g128_int4_mfma(gpu, M, K, parts, unroll):
     for batch in (1, 5, 16):
         p = gen.int4_problem(M, K, 128, batch=batch, seed=K + batch + parts)
