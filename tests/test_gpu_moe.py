@@ -13,7 +13,7 @@ import torch
 
 import oracle
 from kernels_amd import gen, kq
-from tests._util import assert_close, dev, host_bits, inf_rel, to_f64
+from tests._util import assert_close, dev, host_bits, inf_rel, moe_gate_up_partitions, to_f64
 
 pytestmark = pytest.mark.gpu
 GOLD = os.path.join(os.path.dirname(__file__), "golden")
@@ -203,8 +203,9 @@ def test_gate_up_and_down_vs_oracle(gpu, pool16, batch):
                                            (4, 7, "mixed"), (4, 16, "one")])
 def test_standalone_repeated_experts(gpu, slot_pools, tk, batch, kind):
     """A caller's routing that names experts more than once a token: plan
-    entries with up to 128 slots, cut for the partitioned kernels; down with
-    the workspace and without (LDS combine), against the oracle."""
+    entries with up to 128 slots (per-tile and streaming gate/up at these small
+    shapes; down with the workspace, where 128 slots run partitioned with
+    entries cut, and without), against the oracle."""
     d, host, pool = slot_pools[(256, 8)]
     d = kq.MoEDesc(**{**d.as_dict(), "top_k": tk})
     rng = np.random.default_rng(tk * batch)
@@ -227,22 +228,32 @@ def test_standalone_repeated_experts(gpu, slot_pools, tk, batch, kind):
         assert_close(to_f64(b.y), Yref, atol=1e-4, rtol=1e-4, what=f"down {wsb}")
 
 
-# A caller's routing with every expert shared and named twice a token, at
-# shapes that the partitioned gate/up takes (test_routes.py): the plan from idx
-# with entries cut to a token's slots, x of one to four chunks a lane.
-@pytest.mark.parametrize("hidden,inter,ne,tk,batch", [(3072, 512, 8, 8, 16), (4096, 512, 8, 8, 12),
+# A caller's routing that names experts more than once a token, at shapes that the
+# partitioned kernels take (gate/up: asserted; down with a workspace, past
+# the slots' h that fit one workgroup): the plan from idx with entries cut to at most a slot a
+# token, x of one to four chunks a lane, against the oracle.
+@pytest.mark.parametrize("hidden,inter,ne,tk,batch", [(4096, 512, 8, 8, 12), (3072, 576, 8, 8, 16),
                                                       (1024, 1024, 8, 8, 16), (1536, 2048, 12, 4, 9)])
-def test_standalone_gate_up_partitioned_repeats(gpu, hidden, inter, ne, tk, batch):
+def test_standalone_partitioned_repeats(gpu, hidden, inter, ne, tk, batch):
     d, off = _compact_desc(hidden, inter, ne, tk)
+    assert moe_gate_up_partitions(d, batch)
     host = gen.moe_pool(ne, seed=hidden, quantize=True, hidden=hidden, inter=inter, blob=d.blob, off=off)
     rng = np.random.default_rng(batch)
     idx = rng.integers(0, ne, (batch, tk)).astype(np.uint32)
     idx[0] = 3
     X = gen.f16_bits(rng.normal(0, 1, (batch, hidden)))
     b = Block(gpu, d, batch)
-    kq.moe_gate_up_swiglu(dev(host, gpu), d, dev(idx, gpu), dev(X, gpu), b.H, b.ws, b.wsb, batch=batch)
+    pool, idx_d = dev(host, gpu), dev(idx, gpu)
+    kq.moe_gate_up_swiglu(pool, d, idx_d, dev(X, gpu), b.H, b.ws, b.wsb, batch=batch)
     torch.cuda.synchronize()
     assert_close(to_f64(b.H), oracle.moe_gate_up(host, odesc(d), idx, X, oracle.F16, batch), what="h")
+    wgt = rng.dirichlet(np.ones(tk), batch).astype(np.float32)
+    Yref = oracle.moe_down(host, odesc(d), idx, wgt.astype(np.float64), host_bits(b.H, np.uint16), batch)
+    for ws, wsb in ((b.ws, b.wsb), (None, 0)):
+        b.y.fill_(float("nan"))
+        kq.moe_down_combine(pool, d, idx_d, torch.from_numpy(wgt).to(gpu), b.H, b.y, ws, wsb, batch=batch)
+        torch.cuda.synchronize()
+        assert_close(to_f64(b.y), Yref, atol=1e-4, rtol=1e-4, what=f"down {wsb}")
 
 
 def test_duplicate_and_shared_experts(gpu, pool16):
