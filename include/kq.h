@@ -156,7 +156,8 @@ kq_status kq_stream_read_out(const void* src, size_t bytes, uint16_t* out, uint3
  * rows_per_cb = 256 and scale_group = K is the per-row-scale format.
  * Constraints: K % 32 == 0, K <= 30000 (x is staged in LDS, else
  * KQ_EUNSUPPORTED), scale_group == K or a power of two >= 32 dividing K,
- * rows_per_cb >= 1, 1 <= batch <= 16.
+ * rows_per_cb >= 1, 1 <= batch <= 16. C and S are finite: an infinite codeword or
+ * scale gives NaN also where no x multiplies it (K is padded with zeros of x).
  *
  * Replaces: gemv_vq_wide (v5) vq-gemv/src/kernels.metal:337-380, encoded by
  *   addVQ vq-gemv/src/main.mm:266-286,308-312.

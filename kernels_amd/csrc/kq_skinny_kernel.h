@@ -40,7 +40,8 @@
 //     unaligned words, and no word reaches past its row.
 //   * the last pair of a row ends at K (it overlaps the pair before unless
 //     256 divides K, with the k already taken zeroed in x), so every load of
-//     weights and scales lies inside its row for any K >= 256.
+//     weights and scales lies inside its row for any K >= 256. (An infinite
+//     codeword or scale would meet those zeros and give NaN.)
 //
 // Work split: a workgroup of P x Q waves owns tiles_wg row tiles; wave (p, q)
 // takes K part p (J pairs) of tiles (round * Q + q) * T ..., T at a time, and

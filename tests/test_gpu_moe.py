@@ -230,8 +230,8 @@ def test_standalone_repeated_experts(gpu, slot_pools, tk, batch, kind):
 
 # A caller's routing that names experts more than once a token, at shapes that the
 # partitioned kernels take (gate/up: asserted; down with a workspace, past
-# the slots' h that fit one workgroup): the plan from idx with entries cut to at most a slot a
-# token, x of one to four chunks a lane, against the oracle.
+# the slots' h that fit one workgroup): the plan from idx with entries cut to at
+# most as many slots as tokens, x of one to four chunks a lane, against the oracle.
 @pytest.mark.parametrize("hidden,inter,ne,tk,batch", [(4096, 512, 8, 8, 12), (3072, 576, 8, 8, 16),
                                                       (1024, 1024, 8, 8, 16), (1536, 2048, 12, 4, 9)])
 def test_standalone_partitioned_repeats(gpu, hidden, inter, ne, tk, batch):
